@@ -1,8 +1,9 @@
 // General-shape paged attention, and the partition combine.
 //
-// Serves every shape the MFMA kernels do not: fp32 pools (whose parity bar is
-// 1e-5, so the arithmetic stays fp32 throughout), any head_dim up to 512 and
-// any number of query heads per KV head. It is the same attention as
+// Serves every shape the MFMA kernels do not: any head_dim up to 512, any
+// number of query heads per KV head, rows of any alignment, in fp32
+// arithmetic throughout (fp32 pools of head_dim 64 or 128 run in
+// attend_f32.hip). It is the same attention as
 // liteinfer's Triton body (liteinfer/models/paged_kernels.py:216-371): an
 // online softmax folded over key tiles, m' = max(m, rowmax(s)),
 // acc = acc * e^(m - m') + e^(s - m') V, l = l * e^(m - m') + sum e^(s - m'),

@@ -173,6 +173,12 @@ constexpr int kMfmaMaxHeadDim = 128;
 int launch_attend_generic(const AttnArgs& a, int dtype, hipStream_t s);
 int launch_combine(const AttnArgs& a, int dtype, hipStream_t s);
 
+// fp32 pools on the fp32 matrix cores (attend_f32.hip): head_dim 64 or 128,
+// every row 16-byte aligned; decode partitions (combined by launch_combine)
+// and packed passes alike.
+bool attend_f32_applies(const AttnArgs& a, int dtype);
+int launch_attend_f32(AttnArgs a, hipStream_t s);
+
 // MFMA decode: bf16 / fp16, head_dim 64 or 128, up to 16 query heads per KV
 // head, every row 16-byte aligned. Returns LI_EUNSUPPORTED when not
 // applicable (nothing launched).

@@ -346,7 +346,8 @@ int paged_decode_impl(const void* q, int64_t q_stride_seq, int64_t q_stride_head
     set_balanced(a, waves, workspace);
     return launch_decode_mfma(a, dtype, s);
   }
-  int rc = mfma ? launch_decode_mfma(a, dtype, s) : launch_attend_generic(a, dtype, s);
+  const bool f32 = !(flags & LI_FLAG_FORCE_GENERIC) && attend_f32_applies(a, dtype);
+  int rc = mfma ? launch_decode_mfma(a, dtype, s) : f32 ? launch_attend_f32(a, s) : launch_attend_generic(a, dtype, s);
   if (rc) return rc;
   if (parts > 1) rc = launch_combine(a, dtype, s);
   return rc;
@@ -628,6 +629,7 @@ int paged_prefill_impl(const void* q, int64_t q_stride_tok, int64_t q_stride_hea
     a.single_query_elsewhere = 1;
     return launch_prefill_mfma(a, dtype, s);
   }
+  if (!(flags & LI_FLAG_FORCE_GENERIC) && attend_f32_applies(a, dtype)) return launch_attend_f32(a, s);
   a.block_q = block_q > 0 ? block_q : 16;
   a.num_qblocks = cdiv(max_query_len, a.block_q);
   return launch_attend_generic(a, dtype, s);

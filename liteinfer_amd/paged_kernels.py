@@ -18,8 +18,8 @@ C-ABI library in ``csrc/`` on torch's current stream:
   call.
 
 bf16/fp16 pools with head_dim 64 or 128 and up to 16 query heads per KV head
-run on the MFMA kernels; every other shape (fp32 above all) on a
-general-shape kernel with fp32 arithmetic. Nothing here has a CPU fallback:
+run on the MFMA kernels, fp32 pools with head_dim 64 or 128 on the fp32 matrix
+cores; every other shape on a general-shape kernel with fp32 arithmetic. Nothing here has a CPU fallback:
 without the HIP library, or off a ROCm device, the calls raise.
 """
 

@@ -1,0 +1,77 @@
+"""fp32 attention on the fp32 matrix cores (head_dim 64 and 128) against the fp64 oracle.
+
+Sizes sit at the kernel's edges: 16-key tiles, 16-row groups and blocks of
+32 rows (with groupings that fill them oddly), a single key, more keys than
+four waves' tiles, pinned splits, and rows whose block reaches past keys they
+do not see. Bound: fp32's 1e-5 (the sums run over at most a few thousand
+products of N(0, 1) values, ~1e-6 off).
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from liteinfer_amd.paged_kernels import paged_decode, paged_prefill
+from tests.helpers import PagedBatch, to_numpy
+
+pytestmark = pytest.mark.gpu
+
+
+def _prefill(b, **kw):
+    return paged_prefill(b.query, b.key_pool, b.value_pool, b.slot_table, b.context_lens_t, b.query_start_loc,
+                         max(b.query_lens), b.scaling, b.groups, **kw)
+
+
+def _close(actual, expected):
+    np.testing.assert_allclose(to_numpy(actual), expected, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("groups", [1, 4, 5, 16, 20])
+@pytest.mark.parametrize("num_splits", [None, 3])
+def test_decode(head_dim, groups, num_splits):
+    b = PagedBatch([1, 15, 16, 17, 63, 64, 65, 1000, 2500], num_heads=3 * groups, num_kv_heads=3, head_dim=head_dim)
+    _close(paged_decode(b.query, b.key_pool, b.value_pool, b.slot_table, b.context_lens_t, b.scaling, b.groups,
+                        num_splits=num_splits), b.oracle())
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("groups", [1, 3, 4, 16, 20])
+def test_packed(head_dim, groups):
+    q = [1, 2, 4, 8, 9, 16, 17, 33, 100, 1]
+    ctx = [1, 2, 90, 8, 25, 300, 17, 64, 163, 700]
+    b = PagedBatch(ctx, q, num_heads=2 * groups, num_kv_heads=2, head_dim=head_dim)
+    _close(_prefill(b), b.oracle())
+    # Through strided rows (the packed boundary's transposed query) too.
+    wide = torch.randn(b.query.shape[1], b.query.shape[0], head_dim, device="cuda").copy_(b.query.transpose(0, 1))
+    strided = paged_prefill(wide.transpose(0, 1), b.key_pool, b.value_pool, b.slot_table, b.context_lens_t,
+                            b.query_start_loc, max(q), b.scaling, b.groups)
+    assert torch.equal(strided, _prefill(b))
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_a_row_is_not_touched_by_values_it_does_not_see(value):
+    """A later token's V row holds an infinity or a NaN: earlier rows stay what they were."""
+    b = PagedBatch([70, 40], [30, 40], num_heads=8, num_kv_heads=2, head_dim=64)
+    b.slot_table = torch.arange(140, device="cuda").reshape(2, 70)  # a slot per position
+    want = _prefill(b)
+    b.value_pool[60] = value  # position 60 of sequence 0: its queries are positions 40 .. 69
+    got = _prefill(b)
+    assert torch.equal(got[:20], want[:20]) or torch.allclose(got[:20], want[:20], rtol=1e-5, atol=1e-5)
+    assert not torch.isfinite(got[20:30]).any()
+    assert torch.equal(got[30:], want[30:])
+
+
+def test_an_unaligned_row_takes_the_general_kernel():
+    b = PagedBatch([40, 90], head_dim=64)
+    odd = torch.zeros(b.query.numel() + 1, device="cuda")[1:].view(b.query.shape).copy_(b.query)
+    _close(paged_decode(odd, b.key_pool, b.value_pool, b.slot_table, b.context_lens_t, b.scaling, b.groups), b.oracle())
+
+
+def test_an_empty_context_is_nan():
+    b = PagedBatch([5, 9], head_dim=64)
+    lens = torch.tensor([0, 9], dtype=torch.int32, device="cuda")
+    out = paged_decode(b.query, b.key_pool, b.value_pool, b.slot_table, lens, b.scaling, b.groups)
+    assert torch.isnan(out[0]).all() and torch.isfinite(out[1]).all()
