@@ -414,6 +414,36 @@ int li_silu_mul(const void* gate_up, void* out, int64_t rows, int ffn,
                 int64_t gate_up_stride, int64_t out_stride, int dtype,
                 void* stream);
 
+/*
+ * The engine's projections at a decode step's batch (torch GEMMs in larger
+ * passes): out = x w^T for x [m, k] (m <= LI_SKINNY_MAX_ROWS) and w [n, k]
+ * (bf16 / fp16 rows 16-byte aligned, last axis contiguous, strides in
+ * elements; n a multiple of 8, k of 128), products summed in fp32.
+ *
+ * li_skinny_gemm_plan reports the runs of k the call should be cut into to
+ * fill the GPU (*splits), or LI_EUNSUPPORTED. With splits == 1 `out` receives
+ * the rounded rows; otherwise `partials`, [splits, m, n] fp32, the sums of
+ * each run, for one of the *_partials calls (which add and round them as
+ * their delta / gate_up) or li_skinny_reduce (which rounds them to rows).
+ * gate_up != 0: w holds [gate | up] rows, n / 2 each; out is then
+ * silu(gate) * up, n / 2 wide (partials: the plain sums).
+ */
+#define LI_SKINNY_MAX_ROWS 64
+int li_skinny_gemm_plan(int m, int n, int k, int* splits);
+int li_skinny_gemm(const void* x, int64_t x_stride, const void* w,
+                   int64_t w_stride, void* out, int64_t out_stride,
+                   float* partials, int m, int n, int k, int splits,
+                   int gate_up, int dtype, void* stream);
+int li_skinny_reduce(const float* partials, void* out, int64_t out_stride,
+                     int m, int n, int splits, int dtype, void* stream);
+int li_add_rms_norm_partials(void* h, const float* partials, int splits,
+                             const void* weight, void* out, int64_t rows,
+                             int hidden, int64_t h_stride, int64_t out_stride,
+                             float eps, int dtype, void* stream);
+int li_silu_mul_partials(const float* partials, int splits, void* out,
+                         int64_t rows, int ffn, int64_t out_stride, int dtype,
+                         void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -54,6 +54,11 @@ EXPORTED_SYMBOLS = (
     "li_paged_prefill_ex",
     "li_add_rms_norm",
     "li_silu_mul",
+    "li_skinny_gemm_plan",
+    "li_skinny_gemm",
+    "li_skinny_reduce",
+    "li_add_rms_norm_partials",
+    "li_silu_mul_partials",
 )
 
 _i64, _i32, _p, _f32, _sz = ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_float, ctypes.c_size_t
@@ -62,6 +67,11 @@ _i64p = ctypes.POINTER(ctypes.c_int64)
 _SIGNATURES = {
     "li_add_rms_norm": (_i32, [_p, _p, _p, _p, _i64, _i32, _i64, _i64, _i64, _f32, _i32, _p]),
     "li_silu_mul": (_i32, [_p, _p, _i64, _i32, _i64, _i64, _i32, _p]),
+    "li_skinny_gemm_plan": (_i32, [_i32, _i32, _i32, ctypes.POINTER(_i32)]),
+    "li_skinny_gemm": (_i32, [_p, _i64, _p, _i64, _p, _i64, _p, _i32, _i32, _i32, _i32, _i32, _i32, _p]),
+    "li_skinny_reduce": (_i32, [_p, _p, _i64, _i32, _i32, _i32, _i32, _p]),
+    "li_add_rms_norm_partials": (_i32, [_p, _p, _i32, _p, _p, _i64, _i32, _i64, _i64, _f32, _i32, _p]),
+    "li_silu_mul_partials": (_i32, [_p, _i32, _p, _i64, _i32, _i64, _i32, _p]),
     "li_last_error_string": (ctypes.c_char_p, []),
     "li_abi_version": (_i32, []),
     "li_build_id": (ctypes.c_char_p, []),

@@ -21,11 +21,14 @@ struct Vec8 {
 constexpr int kNormPer = 4;
 
 // h <- h + delta (when delta is given), rounded to T; out <- weight *
-// T(h * rsqrt(mean(h^2) + eps)), the product rounded to T.
+// T(h * rsqrt(mean(h^2) + eps)), the product rounded to T. With `splits` > 0
+// delta is a projection's fp32 sums over as many runs of its K
+// ([splits][rows][hidden], skinny_gemm.hip), added here and rounded to T: one
+// launch less than rounding them on their own.
 template <typename T>
 __global__ __launch_bounds__(kNormThreads) void add_rms_norm(T* h, const T* delta, const T* weight, T* out,
                                                             int hidden, int64_t h_s, int64_t d_s, int64_t o_s,
-                                                            float eps) {
+                                                            float eps, const float* part, int splits) {
   typedef typename Vec8<T>::type V;
   const int64_t row = blockIdx.x;
   T* hrow = h + row * h_s;
@@ -43,6 +46,29 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm(T* h, const T* delt
         const V dv = *reinterpret_cast<const V*>(drow + 8 * c);
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = li_from_float<T>((float)v[e] + (float)dv[e]);
+        *reinterpret_cast<V*>(hrow + 8 * c) = v;
+      } else if (splits > 0) {
+        float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        for (int p0 = 0; p0 < splits; p0 += 8) {  // eight runs' loads together
+          floatx4_t lo[8], hi[8];
+#pragma unroll
+          for (int u = 0; u < 8; ++u) {
+            const float* src = part + ((int64_t)min(p0 + u, splits - 1) * gridDim.x + row) * hidden + 8 * c;
+            lo[u] = *reinterpret_cast<const floatx4_t*>(src);
+            hi[u] = *reinterpret_cast<const floatx4_t*>(src + 4);
+          }
+#pragma unroll
+          for (int u = 0; u < 8; ++u)
+            if (p0 + u < splits) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                sum[e] += lo[u][e];
+                sum[4 + e] += hi[u][e];
+              }
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = li_from_float<T>((float)v[e] + (float)li_from_float<T>(sum[e]));
         *reinterpret_cast<V*>(hrow + 8 * c) = v;
       }
 #pragma unroll
@@ -78,16 +104,42 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm(T* h, const T* delt
 
 // out[r, i] = T(T(silu(gate)) * up) with gate = gu[r, i], up = gu[r, F + i]
 // (torch's F.silu(gate) * up on the two halves of the fused projection).
+// With `splits` > 0 the projection is given as its fp32 sums over as many
+// runs of K, [splits][rows][2 F], added and rounded to T first.
 template <typename T>
-__global__ __launch_bounds__(256) void silu_mul(const T* gu, T* out, int64_t rows, int f, int64_t gu_s, int64_t o_s) {
+__global__ __launch_bounds__(256) void silu_mul(const T* gu, T* out, int64_t rows, int f, int64_t gu_s, int64_t o_s,
+                                                const float* part, int splits) {
   typedef typename Vec8<T>::type V;
   const int chunks = f / 8;
   const int64_t total = rows * chunks;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
     const int64_t r = i / chunks;
     const int c = (int)(i - r * chunks);
-    const V g = *reinterpret_cast<const V*>(gu + r * gu_s + 8 * c);
-    const V u = *reinterpret_cast<const V*>(gu + r * gu_s + f + 8 * c);
+    V g, u;
+    if (splits > 0) {
+      float gs[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, us[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      for (int p = 0; p < splits; ++p) {
+        const float* src = part + ((int64_t)p * rows + r) * 2 * f + 8 * c;
+#pragma unroll
+        for (int e = 0; e < 8; e += 4) {
+          const floatx4_t gv = *reinterpret_cast<const floatx4_t*>(src + e);
+          const floatx4_t uv = *reinterpret_cast<const floatx4_t*>(src + f + e);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            gs[e + q] += gv[q];
+            us[e + q] += uv[q];
+          }
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        g[e] = li_from_float<T>(gs[e]);
+        u[e] = li_from_float<T>(us[e]);
+      }
+    } else {
+      g = *reinterpret_cast<const V*>(gu + r * gu_s + 8 * c);
+      u = *reinterpret_cast<const V*>(gu + r * gu_s + f + 8 * c);
+    }
     V o;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -105,49 +157,80 @@ bool rows_ok(const void* p, int64_t stride, int esize) {
 
 }  // namespace
 
-extern "C" int li_add_rms_norm(void* h, const void* delta, const void* weight, void* out, int64_t rows, int hidden,
-                               int64_t h_stride, int64_t delta_stride, int64_t out_stride, float eps, int dtype,
-                               void* stream) {
+namespace {
+
+int add_rms_norm_impl(const char* who, void* h, const void* delta, const float* partials, int splits, const void* weight,
+                      void* out, int64_t rows, int hidden, int64_t h_stride, int64_t delta_stride, int64_t out_stride,
+                      float eps, int dtype, void* stream) {
   li::clear_error();
-  if (dtype != LI_BF16 && dtype != LI_F16) return li::fail(LI_EUNSUPPORTED, "li_add_rms_norm: bf16 or f16 rows only");
+  if (dtype != LI_BF16 && dtype != LI_F16) return li::fail(LI_EUNSUPPORTED, "%s: bf16 or f16 rows only", who);
   if (rows < 0 || hidden <= 0 || hidden % 8 != 0 || hidden > 8 * kNormThreads * kNormPer)
-    return li::fail(LI_EINVAL, "li_add_rms_norm: hidden size %d must be a multiple of 8 up to %d", hidden,
+    return li::fail(LI_EINVAL, "%s: hidden size %d must be a multiple of 8 up to %d", who, hidden,
                     8 * kNormThreads * kNormPer);
   if (rows == 0) return LI_OK;
-  if (rows > 0x7fffffffLL) return li::fail(LI_EINVAL, "li_add_rms_norm: too many rows");
+  if (rows > 0x7fffffffLL) return li::fail(LI_EINVAL, "%s: too many rows", who);
   if (!h || !weight || !out || !rows_ok(h, h_stride, 2) || !rows_ok(out, out_stride, 2) || !li::aligned16(weight) ||
-      (delta && !rows_ok(delta, delta_stride, 2)))
-    return li::fail(LI_EINVAL, "li_add_rms_norm: rows must be 16-byte aligned with the last axis contiguous");
+      (delta && !rows_ok(delta, delta_stride, 2)) || (splits > 0 && (!partials || !li::aligned16(partials))))
+    return li::fail(LI_EINVAL, "%s: rows must be 16-byte aligned with the last axis contiguous", who);
   hipStream_t s = static_cast<hipStream_t>(stream);
   const dim3 g((unsigned)rows), b(kNormThreads);
   if (dtype == LI_BF16)
     hipLaunchKernelGGL(add_rms_norm<li_bf16>, g, b, 0, s, static_cast<li_bf16*>(h), static_cast<const li_bf16*>(delta),
                        static_cast<const li_bf16*>(weight), static_cast<li_bf16*>(out), hidden, h_stride,
-                       delta_stride, out_stride, eps);
+                       delta_stride, out_stride, eps, partials, splits);
   else
     hipLaunchKernelGGL(add_rms_norm<li_f16>, g, b, 0, s, static_cast<li_f16*>(h), static_cast<const li_f16*>(delta),
                        static_cast<const li_f16*>(weight), static_cast<li_f16*>(out), hidden, h_stride, delta_stride,
-                       out_stride, eps);
-  return li::check_launch("li_add_rms_norm");
+                       out_stride, eps, partials, splits);
+  return li::check_launch(who);
 }
 
-extern "C" int li_silu_mul(const void* gate_up, void* out, int64_t rows, int ffn, int64_t gate_up_stride,
-                           int64_t out_stride, int dtype, void* stream) {
+int silu_mul_impl(const char* who, const void* gate_up, const float* partials, int splits, void* out, int64_t rows,
+                  int ffn, int64_t gate_up_stride, int64_t out_stride, int dtype, void* stream) {
   li::clear_error();
-  if (dtype != LI_BF16 && dtype != LI_F16) return li::fail(LI_EUNSUPPORTED, "li_silu_mul: bf16 or f16 rows only");
-  if (rows < 0 || ffn <= 0 || ffn % 8 != 0) return li::fail(LI_EINVAL, "li_silu_mul: ffn %d must be a multiple of 8", ffn);
+  if (dtype != LI_BF16 && dtype != LI_F16) return li::fail(LI_EUNSUPPORTED, "%s: bf16 or f16 rows only", who);
+  if (rows < 0 || ffn <= 0 || ffn % 8 != 0) return li::fail(LI_EINVAL, "%s: ffn %d must be a multiple of 8", who, ffn);
   if (rows == 0) return LI_OK;
-  if (!gate_up || !out || !rows_ok(gate_up, gate_up_stride, 2) || !rows_ok(out, out_stride, 2) || (ffn * 2) % 16)
-    return li::fail(LI_EINVAL, "li_silu_mul: rows must be 16-byte aligned with the last axis contiguous");
+  if ((splits > 0 ? !partials || !li::aligned16(partials) : !gate_up || !rows_ok(gate_up, gate_up_stride, 2)) || !out ||
+      !rows_ok(out, out_stride, 2) || (ffn * 2) % 16)
+    return li::fail(LI_EINVAL, "%s: rows must be 16-byte aligned with the last axis contiguous", who);
   const int64_t work = rows * (ffn / 8);
   const int64_t blocks = std::min<int64_t>(li::cdiv64(work, 256), 65536);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == LI_BF16)
     hipLaunchKernelGGL(silu_mul<li_bf16>, dim3((unsigned)blocks), dim3(256), 0, s,
                        static_cast<const li_bf16*>(gate_up), static_cast<li_bf16*>(out), rows, ffn, gate_up_stride,
-                       out_stride);
+                       out_stride, partials, splits);
   else
     hipLaunchKernelGGL(silu_mul<li_f16>, dim3((unsigned)blocks), dim3(256), 0, s, static_cast<const li_f16*>(gate_up),
-                       static_cast<li_f16*>(out), rows, ffn, gate_up_stride, out_stride);
-  return li::check_launch("li_silu_mul");
+                       static_cast<li_f16*>(out), rows, ffn, gate_up_stride, out_stride, partials, splits);
+  return li::check_launch(who);
+}
+
+}  // namespace
+
+extern "C" int li_add_rms_norm(void* h, const void* delta, const void* weight, void* out, int64_t rows, int hidden,
+                               int64_t h_stride, int64_t delta_stride, int64_t out_stride, float eps, int dtype,
+                               void* stream) {
+  return add_rms_norm_impl("li_add_rms_norm", h, delta, nullptr, 0, weight, out, rows, hidden, h_stride, delta_stride,
+                           out_stride, eps, dtype, stream);
+}
+
+extern "C" int li_add_rms_norm_partials(void* h, const float* partials, int splits, const void* weight, void* out,
+                                        int64_t rows, int hidden, int64_t h_stride, int64_t out_stride, float eps,
+                                        int dtype, void* stream) {
+  if (splits < 1) return li::fail(LI_EINVAL, "li_add_rms_norm_partials: %d splits", splits);
+  return add_rms_norm_impl("li_add_rms_norm_partials", h, nullptr, partials, splits, weight, out, rows, hidden, h_stride,
+                           0, out_stride, eps, dtype, stream);
+}
+
+extern "C" int li_silu_mul(const void* gate_up, void* out, int64_t rows, int ffn, int64_t gate_up_stride,
+                           int64_t out_stride, int dtype, void* stream) {
+  return silu_mul_impl("li_silu_mul", gate_up, nullptr, 0, out, rows, ffn, gate_up_stride, out_stride, dtype, stream);
+}
+
+extern "C" int li_silu_mul_partials(const float* partials, int splits, void* out, int64_t rows, int ffn,
+                                    int64_t out_stride, int dtype, void* stream) {
+  if (splits < 1) return li::fail(LI_EINVAL, "li_silu_mul_partials: %d splits", splits);
+  return silu_mul_impl("li_silu_mul_partials", nullptr, partials, splits, out, rows, ffn, 0, out_stride, dtype, stream);
 }

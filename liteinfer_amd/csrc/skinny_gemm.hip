@@ -1,0 +1,275 @@
+// out = x W^T for few rows of x (a decode step's batch): the engine's
+// projections, q/k/v, output, gate/up with the SiLU gate, down and head
+// (liteinfer/models/llama.py:101-161, nn.Linear in the reference).
+//
+// At a decode step's batch a projection reads its weights once and does
+// little else, so its bound is HBM: x is a few hundred KB and stays in L2.
+// A work-group of NW waves takes a tile of 16 NW weight rows (N) and a run
+// of K, all BM rows of x beside it. Both operands go straight into LDS
+// (global_load_lds_dwordx4) in a ring of stages of 128 k: rows of 256 bytes,
+// 16-byte chunk c of row r at c ^ (r % 16), so that the 16 rows an operand
+// read spans lie in 16 different bank groups. R - 1 stages are in flight, one
+// barrier a stage; up to 32 rows two work-groups of four waves share a CU
+// (96 .. 120 KiB in flight on it; 27 GB/s a CU times ~2 us of loaded latency
+// needs ~54), past that one of eight. Wave w owns weight rows 16 w .. + 15:
+//   D (16 n x 16 m) += A = W rows (16 n x 32 k), B = x^T (32 k x 16 m)
+// and lane (m, g) = (lane % 16, lane / 16) ends with outputs n = 4g .. 4g + 3
+// of row m. Sums are fp32, rounded once.
+//
+// Few tiles are cut along K into `splits` runs so that the grid fills the GPU;
+// each run then writes its fp32 sums and the op that follows (add_rms_norm,
+// silu_mul or skinny_reduce) adds them before it rounds.
+//
+// Where a work-group starts its run of K matters: rows of a power-of-two
+// stride read at one k at a time by every work-group of an XCD meet on a few
+// HBM channels. The stages are taken in a rotated order, five further for
+// each work-group an XCD holds (gate/up of the 8B architecture, one row: 44.8
+// us unrotated, 36.9 rotated, 39 .. 42 rotated by the tile itself).
+//
+// Measured (MI355X, graph replay over weights larger than the caches), rows 1
+// and 32, us (TB/s of weights at one row), against hipBLASLt's:
+//   6144 x 4096    10.1 (5.0)  11.3      14.5  15.3
+//   4096 x 4096     7.6 (4.4)   8.5      15.4  13.1
+//   28672 x 4096   39.0 (6.0)  40.7      66.3  57.8   (the gate included)
+//   4096 x 14336   20.5 (5.7)  22.4      27.2  31.5
+//   16032 x 4096   22.3 (5.9)  23.7      29.4  27.5
+//   2048 x 2048     3.6 (2.3)   4.8      11.0  11.2
+// The small ones are a launch and one loaded latency.
+#include "li_mfma.h"
+
+namespace {
+
+using namespace li;
+
+constexpr int kStageK = 128;
+constexpr int kRotate = 5;
+constexpr int kRowBytes = kStageK * 2;
+
+struct GemmArgs {
+  const char* x;
+  const char* w;
+  char* out;       // T rows (splits == 1)
+  float* part;     // [splits][m][n] fp32 (splits > 1)
+  int64_t x_s, w_s, o_s;  // row strides in bytes (x, w), in elements (out)
+  int m, n, k;
+  int splits;
+  int gate;  // W holds [gate | up] rows, n / 2 each; out = silu(gate) * up, n / 2 wide
+};
+
+// Weight rows of a work-group's tile at m rows of x, and the work-groups of it
+// a CU holds.
+constexpr int kFewRows = 32;
+int tile_of(int m) { return m <= kFewRows ? 64 : 128; }
+int per_cu(int m) { return m <= kFewRows ? 2 : 1; }
+
+// BM: rows of x a work-group holds (m <= BM). R: ring stages.
+template <typename T, int BM, int R, int NW, bool kGate>
+__global__ __launch_bounds__(64 * NW) void skinny_gemm(GemmArgs a) {
+  using M = Mfma<T>;
+  using Frag = typename M::Frag;
+  constexpr int kMt = BM / 16;
+  constexpr int kTileN = 16 * NW;
+  constexpr int kXPer = BM / 4 / NW;  // x loads of a wave per stage
+  static_assert(kXPer >= 1 && kXPer * 4 * NW == BM, "the waves split x's loads evenly");
+  constexpr int kPer = 4 + kXPer;
+  constexpr int kStage = (kTileN + BM) * kRowBytes;
+  static_assert(R == 3 || R == 4, "the waits below count up to two newer stages");
+  static_assert((R - 2) * kPer < 64, "vmcnt range");
+  __shared__ __attribute__((aligned(1024))) char ring[R][kStage];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n16 = lane & 15, g = lane >> 4;
+  const int tile = (int)(blockIdx.x / (unsigned)a.splits), split = (int)(blockIdx.x % (unsigned)a.splits);
+  const int total = a.k / kStageK;
+  const int s0 = (int)((int64_t)total * split / a.splits), s1 = (int)((int64_t)total * (split + 1) / a.splits);
+  const int ns = s1 - s0;
+
+  // This lane's chunk of the rows it loads: load i of the wave covers four
+  // rows, 16 lanes side by side on each. (Rows past the last repeat it.)
+  const char* wrow[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int t = 4 * i + g;  // row of the wave's 16
+    int64_t row;
+    if (kGate) {  // rows 0-7: gate, 8-15: the up rows of the same outputs
+      const int col = min(tile * (kTileN / 2) + 8 * w + (t & 7), a.n / 2 - 1);
+      row = (t < 8 ? 0 : a.n / 2) + col;
+    } else {
+      row = min(tile * kTileN + 16 * w + t, a.n - 1);
+    }
+    wrow[i] = a.w + row * a.w_s + (int64_t)s0 * kRowBytes + 16 * (n16 ^ t);
+  }
+  const char* xrow[kXPer];
+  int xat[kXPer];
+#pragma unroll
+  for (int i = 0; i < kXPer; ++i) {
+    const int p = w * kXPer + i;  // four-row group of x
+    const int t = 4 * p + g;
+    xrow[i] = a.x + (int64_t)min(t, a.m - 1) * a.x_s + (int64_t)s0 * kRowBytes + 16 * (n16 ^ (t & 15));
+    xat[i] = kTileN * kRowBytes + 1024 * p;
+  }
+  const uint32_t base = lds_addr(&ring[0][0]);
+  const unsigned rotated = (unsigned)(tile >> 3) * kRotate;
+  auto issue = [&](int st) {
+    const uint32_t dst = base + (uint32_t)(st % R) * kStage;
+    const int64_t at = (int64_t)((rotated + (unsigned)st) % (unsigned)ns) * kRowBytes;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dma16<true>(wrow[i] + at, dst + 4096 * w + 1024 * i);
+#pragma unroll
+    for (int i = 0; i < kXPer; ++i) dma16<false>(xrow[i] + at, dst + xat[i]);
+  };
+
+  floatx4_t acc[kMt];
+#pragma unroll
+  for (int i = 0; i < kMt; ++i) acc[i] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  uint32_t off[kStageK / 32];
+#pragma unroll
+  for (int j = 0; j < kStageK / 32; ++j) off[j] = (uint32_t)(n16 * kRowBytes + 16 * ((4 * j + g) ^ n16));
+
+#pragma unroll
+  for (int st = 0; st < R - 1; ++st)
+    if (st < ns) issue(st);
+  for (int st = 0; st < ns; ++st) {
+    // Stage st has landed once only the stages issued after it are in flight.
+    const int newer = min(R - 2, ns - 1 - st);
+    if (newer == 2) li_wait_vm<(R > 3 ? 2 : 1) * kPer>();
+    else if (newer == 1) li_wait_vm<kPer>();
+    else li_wait_vm<0>();
+    lds_barrier();  // every wave's part of it; and all are done with stage st - 1, whose place the next loads take
+    if (st + R - 1 < ns) issue(st + R - 1);
+    const uint32_t cur = base + (uint32_t)(st % R) * kStage;
+#pragma unroll
+    for (int j = 0; j < kStageK / 32; ++j) {
+      const Frag wf = lds_read_frag<Frag>(cur + 4096 * w + off[j]);
+#pragma unroll
+      for (int i = 0; i < kMt; ++i)
+        acc[i] = M::mma(wf, lds_read_frag<Frag>(cur + kTileN * kRowBytes + 4096 * i + off[j]), acc[i]);
+    }
+    // The stage's reads are complete before the next stage's barrier is reached.
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+  // Lane (m, g): outputs 4g .. 4g + 3 of the wave's 16, row 16 i + m.
+#pragma unroll
+  for (int i = 0; i < kMt; ++i) {
+    const int m = 16 * i + n16;
+    if constexpr (kGate) {
+      // Lanes 0-31 hold gate outputs 0-7, lanes 32-63 the up outputs.
+      const int col = tile * (kTileN / 2) + 8 * w + 4 * (g & 1);
+      float o[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float up = __shfl_xor(acc[i][r], 32, 64);
+        if (a.splits == 1) {
+          const float gf = li_to_float(li_from_float<T>(acc[i][r]));
+          const float s = li_to_float(li_from_float<T>(gf / (1.f + expf(-gf))));
+          o[r] = s * li_to_float(li_from_float<T>(up));
+        }
+      }
+      if (a.splits == 1) {
+        if (g < 2 && m < a.m && col < a.n / 2)
+          *reinterpret_cast<uint2*>(a.out + (m * a.o_s + col) * 2) = uint2{li_pack2<T>(o[0], o[1]), li_pack2<T>(o[2], o[3])};
+      } else if (m < a.m && col < a.n / 2) {
+        *reinterpret_cast<floatx4_t*>(a.part + ((int64_t)split * a.m + m) * a.n + (g < 2 ? 0 : a.n / 2) + col) = acc[i];
+      }
+    } else {
+      const int col = tile * kTileN + 16 * w + 4 * g;
+      if (m >= a.m || col >= a.n) continue;
+      if (a.splits == 1)
+        *reinterpret_cast<uint2*>(a.out + (m * a.o_s + col) * 2) =
+            uint2{li_pack2<T>(acc[i][0], acc[i][1]), li_pack2<T>(acc[i][2], acc[i][3])};
+      else
+        *reinterpret_cast<floatx4_t*>(a.part + ((int64_t)split * a.m + m) * a.n + col) = acc[i];
+    }
+  }
+}
+
+// out = the sum of the splits' fp32 sums, rounded.
+template <typename T>
+__global__ __launch_bounds__(256) void skinny_reduce(const float* part, char* out, int64_t o_s, int m, int n, int splits) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= (int64_t)m * n) return;
+  floatx4_t s = {0.f, 0.f, 0.f, 0.f};
+  for (int p0 = 0; p0 < splits; p0 += 8) {
+    floatx4_t v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      v[u] = p0 + u < splits ? *reinterpret_cast<const floatx4_t*>(part + (int64_t)(p0 + u) * m * n + i)
+                             : floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[e] += v[u][e];
+  }
+  const int64_t row = i / n, col = i - row * n;
+  *reinterpret_cast<uint2*>(out + (row * o_s + col) * 2) = uint2{li_pack2<T>(s[0], s[1]), li_pack2<T>(s[2], s[3])};
+}
+
+template <typename T, int BM, int R, int NW>
+void launch(const GemmArgs& a, hipStream_t s) {
+  const dim3 grid((unsigned)((a.n + 16 * NW - 1) / (16 * NW) * a.splits)), block(64 * NW);
+  if (a.gate) hipLaunchKernelGGL((skinny_gemm<T, BM, R, NW, true>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((skinny_gemm<T, BM, R, NW, false>), grid, block, 0, s, a);
+}
+
+template <typename T>
+void launch_rows(const GemmArgs& a, hipStream_t s) {
+  if (a.m <= 16) launch<T, 16, 4, 4>(a, s);
+  else if (a.m <= kFewRows) launch<T, 32, 3, 4>(a, s);
+  else launch<T, 64, 3, 8>(a, s);
+}
+
+}  // namespace
+
+extern "C" int li_skinny_gemm_plan(int m, int n, int k, int* splits) {
+  li::clear_error();
+  if (m < 0 || n <= 0 || k <= 0) return li::fail(LI_EINVAL, "li_skinny_gemm_plan: bad extents (%d, %d, %d)", m, n, k);
+  if (m > LI_SKINNY_MAX_ROWS || n % 8 || k % kStageK)
+    return li::fail(LI_EUNSUPPORTED, "li_skinny_gemm: up to %d rows, n a multiple of 8, k of %d; got %d, %d, %d",
+                    LI_SKINNY_MAX_ROWS, kStageK, m, n, k);
+  // As many runs of K as fill the GPU once, at least one stage each; none
+  // where the tiles alone are three quarters of a work-group a CU or more
+  // (what a second run gains is less than adding the sums costs: 16,032 x
+  // 4,096 at 8 rows 21.5 us whole, 26.9 in two, 21.4 in four).
+  const int tiles = (n + tile_of(m) - 1) / tile_of(m), cus = li::device_cu_count();
+  const int want = tiles * 4 >= cus * 3 ? 1 : cus * per_cu(m) / tiles;
+  if (splits) *splits = std::max(1, std::min(want, k / kStageK));
+  return LI_OK;
+}
+
+extern "C" int li_skinny_gemm(const void* x, int64_t x_stride, const void* w, int64_t w_stride, void* out,
+                              int64_t out_stride, float* partials, int m, int n, int k, int splits, int gate_up,
+                              int dtype, void* stream) {
+  li::clear_error();
+  if (dtype != LI_BF16 && dtype != LI_F16) return li::fail(LI_EUNSUPPORTED, "li_skinny_gemm: bf16 or f16 only");
+  if (int rc = li_skinny_gemm_plan(m, n, k, nullptr)) return rc;
+  if (splits < 1 || splits > k / kStageK) return li::fail(LI_EINVAL, "li_skinny_gemm: %d splits of %d", splits, k);
+  if (gate_up && n % 16) return li::fail(LI_EUNSUPPORTED, "li_skinny_gemm: gate / up halves must be multiples of 8");
+  if (m == 0) return LI_OK;
+  if (!x || !w || (splits == 1 ? !out : !partials)) return li::fail(LI_EINVAL, "li_skinny_gemm: null pointer");
+  if (!li::aligned16(x) || !li::aligned16(w) || (x_stride * 2) % 16 || (w_stride * 2) % 16 || x_stride < 0 || w_stride < k ||
+      (splits == 1 ? (reinterpret_cast<uintptr_t>(out) % 8 || out_stride % 4) : !li::aligned16(partials)))
+    return li::fail(LI_EINVAL, "li_skinny_gemm: rows must be 16-byte aligned with the last axis contiguous");
+  const GemmArgs a{static_cast<const char*>(x), static_cast<const char*>(w), static_cast<char*>(out), partials,
+                   x_stride * 2, w_stride * 2, out_stride, m, n, k, splits, gate_up};
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (dtype == LI_BF16) launch_rows<li_bf16>(a, s);
+  else launch_rows<li_f16>(a, s);
+  return li::check_launch("li_skinny_gemm");
+}
+
+extern "C" int li_skinny_reduce(const float* partials, void* out, int64_t out_stride, int m, int n, int splits,
+                                int dtype, void* stream) {
+  li::clear_error();
+  if (dtype != LI_BF16 && dtype != LI_F16) return li::fail(LI_EUNSUPPORTED, "li_skinny_reduce: bf16 or f16 only");
+  if (m < 0 || n <= 0 || n % 8 || splits < 1) return li::fail(LI_EINVAL, "li_skinny_reduce: bad extents");
+  if (m == 0) return LI_OK;
+  if (!partials || !out || !li::aligned16(partials) || reinterpret_cast<uintptr_t>(out) % 8 || out_stride % 4)
+    return li::fail(LI_EINVAL, "li_skinny_reduce: null or unaligned pointer");
+  const int64_t work = (int64_t)m * n / 4;
+  const dim3 grid((unsigned)li::cdiv64(work, 256)), block(256);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (dtype == LI_BF16) hipLaunchKernelGGL(skinny_reduce<li_bf16>, grid, block, 0, s, partials, static_cast<char*>(out), out_stride, m, n, splits);
+  else hipLaunchKernelGGL(skinny_reduce<li_f16>, grid, block, 0, s, partials, static_cast<char*>(out), out_stride, m, n, splits);
+  return li::check_launch("li_skinny_reduce");
+}

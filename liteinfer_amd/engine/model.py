@@ -126,13 +126,14 @@ class RandomLlama:
         cos, sin = self._rotary(positions)
         nq, nkv = s.num_heads, s.num_kv_heads
         fused = self._fused_ops
+        linear = fused.linear if fused else F.linear
         delta = None  # the MLP output not yet added to the residual stream
         for idx, layer in enumerate(self.layers):
             if fused:
                 x = fused.add_rms_norm(h, layer.attn_norm, s.rms_norm_eps, delta)
             else:
                 x = self._rms_norm(h, layer.attn_norm)
-            qkv = F.linear(x, layer.w_qkv).view(batch, tokens, nq + 2 * nkv, s.head_dim)
+            qkv = linear(x, layer.w_qkv).view(batch, tokens, nq + 2 * nkv, s.head_dim)
             q = qkv[:, :, :nq].transpose(1, 2)
             k = qkv[:, :, nq:nq + nkv].transpose(1, 2)
             v = qkv[:, :, nq + nkv:].transpose(1, 2)
@@ -140,8 +141,8 @@ class RandomLlama:
             attn = paged_attention(q, kv, self.scaling, s.groups)
             attn = attn.transpose(1, 2).reshape(batch, tokens, nq * s.head_dim)
             if fused:
-                x = fused.add_rms_norm(h, layer.mlp_norm, s.rms_norm_eps, F.linear(attn, layer.w_o))
-                delta = F.linear(fused.silu_mul(F.linear(x, layer.w_gate_up)), layer.w_down)
+                x = fused.add_rms_norm(h, layer.mlp_norm, s.rms_norm_eps, fused.linear_sums(attn, layer.w_o))
+                delta = fused.linear_sums(fused.gate_up_silu(x, layer.w_gate_up), layer.w_down)
             else:
                 h = h + F.linear(attn, layer.w_o)
                 x = self._rms_norm(h, layer.mlp_norm)
@@ -152,4 +153,4 @@ class RandomLlama:
         else:
             h = self._rms_norm(h, self.final_norm)
         rows = h[0, logits_positions] if logits_positions is not None else h[:, -1]
-        return F.linear(rows, self.lm_head)
+        return linear(rows, self.lm_head)

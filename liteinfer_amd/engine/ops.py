@@ -8,7 +8,12 @@ they do not serve (ValueError); the model keeps its torch ops for CPU tensors.
 
 from __future__ import annotations
 
+import ctypes
+import functools
+from typing import NamedTuple
+
 import torch
+import torch.nn.functional as F
 
 from liteinfer_amd import _native
 
@@ -22,13 +27,110 @@ def _rows(t: torch.Tensor, name: str) -> tuple[int, int]:
     return flat.shape[0], (flat.stride(0) if flat.shape[0] > 1 else t.shape[-1])
 
 
-def add_rms_norm(h: torch.Tensor, weight: torch.Tensor, eps: float, delta: torch.Tensor | None = None) -> torch.Tensor:
+class Partials(NamedTuple):
+    """A projection as fp32 sums over runs of its K, ``[splits, rows, n]``: what an op that follows adds and rounds."""
+
+    sums: torch.Tensor
+    shape: torch.Size
+    """The projection's shape, ``[..., n]``."""
+
+
+# Rows of x up to which the projections run as this library's kernel
+# (LI_SKINNY_MAX_ROWS); torch's GEMMs serve larger passes.
+SKINNY_MAX_ROWS = 64
+
+
+@functools.lru_cache(maxsize=4096)
+def _splits(rows: int, n: int, k: int) -> int:
+    """Runs of K one projection is cut into (0: torch's GEMM serves it)."""
+    if rows > SKINNY_MAX_ROWS or n % 8 or k % 128:
+        return 0
+    splits = ctypes.c_int()
+    _native.check(_native.load().li_skinny_gemm_plan(rows, n, k, ctypes.byref(splits)), "skinny_gemm")
+    return splits.value
+
+
+def _skinny(x: torch.Tensor, w: torch.Tensor) -> tuple[torch.Tensor, int]:
+    """x as ``[rows, k]`` and the splits of ``x @ w.T`` (0: not this kernel's)."""
+    flat = x.reshape(-1, x.shape[-1])
+    if (x.dtype not in (torch.bfloat16, torch.float16) or w.dtype != x.dtype or not w.is_contiguous()
+            or flat.stride(-1) != 1 or flat.stride(0) % 8 or flat.data_ptr() % 16 or w.data_ptr() % 16):
+        return flat, 0
+    return flat, _splits(flat.shape[0], *w.shape)
+
+
+def _gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None, sums: torch.Tensor | None, splits: int,
+          gate_up: bool) -> None:
+    status = _native.load().li_skinny_gemm(
+        x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr() if out is not None else None,
+        out.stride(0) if out is not None else 0, sums.data_ptr() if sums is not None else None,
+        x.shape[0], w.shape[0], w.shape[1], splits, int(gate_up), _native.dtype_code(x.dtype),
+        _native.stream_handle(x.device))
+    _native.check(status, "skinny_gemm")
+
+
+def linear_sums(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor | Partials:
+    """``x @ w.T`` for an op that takes `Partials`: those where the kernel cut K, the rounded rows elsewhere."""
+    flat, splits = _skinny(x, w)
+    if splits == 0:
+        return F.linear(x, w)
+    shape = torch.Size((*x.shape[:-1], w.shape[0]))
+    if splits > 1:
+        sums = torch.empty(splits, flat.shape[0], w.shape[0], dtype=torch.float32, device=x.device)
+        _gemm(flat, w, None, sums, splits, False)
+        return Partials(sums, shape)
+    out = torch.empty(flat.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
+    _gemm(flat, w, out, None, 1, False)
+    return out.view(shape)
+
+
+def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """``x @ w.T``, the model's projection."""
+    got = linear_sums(x, w)
+    if not isinstance(got, Partials):
+        return got
+    splits, rows, n = got.sums.shape
+    out = torch.empty(got.shape, dtype=x.dtype, device=x.device)
+    status = _native.load().li_skinny_reduce(got.sums.data_ptr(), out.data_ptr(), n, rows, n, splits,
+                                             _native.dtype_code(x.dtype), _native.stream_handle(x.device))
+    _native.check(status, "skinny_reduce")
+    return out
+
+
+def gate_up_silu(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """``silu(gate) * up`` of the fused projection ``x @ w.T = [gate | up]``."""
+    flat, splits = _skinny(x, w)
+    if splits == 0 or w.shape[0] % 16:
+        return silu_mul(F.linear(x, w))
+    rows, ffn = flat.shape[0], w.shape[0] // 2
+    out = torch.empty(*x.shape[:-1], ffn, dtype=x.dtype, device=x.device)
+    if splits == 1:
+        _gemm(flat, w, out.view(rows, ffn), None, 1, True)
+        return out
+    sums = torch.empty(splits, rows, 2 * ffn, dtype=torch.float32, device=x.device)
+    _gemm(flat, w, None, sums, splits, True)
+    status = _native.load().li_silu_mul_partials(sums.data_ptr(), splits, out.data_ptr(), rows, ffn, ffn,
+                                                 _native.dtype_code(x.dtype), _native.stream_handle(x.device))
+    _native.check(status, "silu_mul")
+    return out
+
+
+def add_rms_norm(h: torch.Tensor, weight: torch.Tensor, eps: float,
+                 delta: torch.Tensor | Partials | None = None) -> torch.Tensor:
     """``h += delta`` in place (when given), then RMSNorm of h times `weight`; returns the normalised rows."""
     if h.dtype not in (torch.bfloat16, torch.float16) or weight.dtype != h.dtype or weight.shape != h.shape[-1:]:
         raise ValueError("add_rms_norm takes bf16 / f16 rows and a weight of their width and dtype")
-    if delta is not None and (delta.shape != h.shape or delta.dtype != h.dtype):
+    if delta is not None and (delta.shape != h.shape or (not isinstance(delta, Partials) and delta.dtype != h.dtype)):
         raise ValueError("delta must match h")
     rows, h_s = _rows(h, "h")
+    if isinstance(delta, Partials):
+        out = torch.empty(h.shape, dtype=h.dtype, device=h.device)
+        status = _native.load().li_add_rms_norm_partials(
+            h.data_ptr(), delta.sums.data_ptr(), delta.sums.shape[0], weight.contiguous().data_ptr(), out.data_ptr(),
+            rows, h.shape[-1], h_s, h.shape[-1], float(eps), _native.dtype_code(h.dtype),
+            _native.stream_handle(h.device))
+        _native.check(status, "add_rms_norm")
+        return out
     d_s = _rows(delta, "delta")[1] if delta is not None else 0
     out = torch.empty(h.shape, dtype=h.dtype, device=h.device)
     status = _native.load().li_add_rms_norm(
