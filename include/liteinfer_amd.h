@@ -421,14 +421,15 @@ int li_silu_mul(const void* gate_up, void* out, int64_t rows, int ffn,
  * elements; n a multiple of 8, k of 128), products summed in fp32.
  *
  * li_skinny_gemm_plan reports the runs of k the call should be cut into to
- * fill the GPU (*splits), or LI_EUNSUPPORTED. With splits == 1 `out` receives
+ * fill the GPU (*splits), or LI_EUNSUPPORTED where a general GEMM is faster
+ * (most shapes past 64 rows). With splits == 1 `out` receives
  * the rounded rows; otherwise `partials`, [splits, m, n] fp32, the sums of
  * each run, for one of the *_partials calls (which add and round them as
  * their delta / gate_up) or li_skinny_reduce (which rounds them to rows).
  * gate_up != 0: w holds [gate | up] rows, n / 2 each; out is then
  * silu(gate) * up, n / 2 wide (partials: the plain sums).
  */
-#define LI_SKINNY_MAX_ROWS 64
+#define LI_SKINNY_MAX_ROWS 256
 int li_skinny_gemm_plan(int m, int n, int k, int* splits);
 int li_skinny_gemm(const void* x, int64_t x_stride, const void* w,
                    int64_t w_stride, void* out, int64_t out_stride,

@@ -1,4 +1,4 @@
-// out = x W^T for few rows of x (a decode step's batch): the engine's
+// out = x W^T for the rows of a decode step's batch: the engine's
 // projections, q/k/v, output, gate/up with the SiLU gate, down and head
 // (liteinfer/models/llama.py:101-161, nn.Linear in the reference).
 //
@@ -56,11 +56,88 @@ struct GemmArgs {
   int gate;  // W holds [gate | up] rows, n / 2 each; out = silu(gate) * up, n / 2 wide
 };
 
-// Weight rows of a work-group's tile at m rows of x, and the work-groups of it
-// a CU holds.
-constexpr int kFewRows = 32;
-int tile_of(int m) { return m <= kFewRows ? 64 : 128; }
-int per_cu(int m) { return m <= kFewRows ? 2 : 1; }
+// Rows of x up to which skinny_gemm runs its small work-groups, and up to
+// which it runs at all (batch_gemm past them).
+constexpr int kFewRows = 32, kSkinnyRows = 64;
+
+// How a projection is cut: weight rows of a tile, runs of K (0: it is left to
+// the caller's own GEMM).
+struct Cut {
+  int tile, splits;
+};
+
+// Up to 64 rows every projection measured faster here than through hipBLASLt
+// (1.0 .. 3.0 times, 10 shapes of the 8B and 1B architectures). K is cut into
+// as many runs as fill the GPU once, at least one stage each; not at all where
+// the tiles alone are three quarters of a work-group a CU or more (what a
+// second run gains is less than adding the sums costs: 16,032 x 4,096 at 8
+// rows 21.5 us whole, 26.9 in two).
+//
+// Past 64 rows a work-group reads x as often as its weights, and the runs'
+// sums cost more than they did; what stays faster (us, this against
+// hipBLASLt's, the norm that adds the sums included):
+//   whole tiles at up to 128 rows: 28672 x 4096 with its gate 53 / 58 at 128
+//     rows (74 / 61 at 160), 32064 x 2048 30 / 34;
+//   runs of K no shorter than 768 of a weight no wider than twice its K:
+//     4096 x 14336 40 / 79 at 128 rows and 49 / 66 at 256, 6144 x 4096 24 / 25
+//     and 30 / 40 (4096 x 4096, runs of 512: 24 / 29 and 28 / 27; 3072 x 2048,
+//     runs of 205: 17 / 14; 16032 x 4096, twice as wide: 38 / 35);
+//   the same in tiles of 64 rows up to 192 rows, half as many runs: 4096 x
+//     4096 22 / 28 at 128 rows, 26 / 31 at 160 (30 / 27 at 256), 2048 x 8192
+//     20 / 24 and 25 / 29.
+constexpr int kMinRun = 768;
+
+Cut cut_of(int m, int n, int k) {
+  const int cus = li::device_cu_count(), stages = k / kStageK;
+  auto tiles = [&](int tile) { return (n + tile - 1) / tile; };
+  auto runs = [&](int tile, int per_cu) {
+    const int t = tiles(tile);
+    return t * 4 >= cus * 3 ? 1 : std::max(1, std::min(cus * per_cu / t, stages));
+  };
+  if (m <= kFewRows) return {64, runs(64, 2)};  // (two work-groups a CU)
+  if (m <= kSkinnyRows) return {128, runs(128, 1)};
+  if (tiles(128) * 4 >= cus * 3) return {128, m <= 128 ? 1 : 0};
+  if (n <= 2 * (int64_t)k) {
+    if (k / runs(128, 1) >= kMinRun) return {128, runs(128, 1)};
+    if (m <= 192 && k / runs(64, 1) >= kMinRun) return {64, runs(64, 1)};
+  }
+  return {0, 0};
+}
+
+// Stores lane (m, g)'s four sums of a group of 16 outputs: 16 group + 4g ..
+// of row m, or with kGate (rows 0-7 of the group: gate outputs 8 group ..,
+// rows 8-15 the up outputs of the same) the gated outputs. Every lane of the
+// wave takes part.
+template <typename T, bool kGate>
+__device__ __forceinline__ void store_outputs(const GemmArgs& a, const floatx4_t& acc, int split, int m, int group,
+                                              int g) {
+  if constexpr (kGate) {
+    // Lanes 0-31 hold gate outputs 0-7, lanes 32-63 the up outputs.
+    const int col = 8 * group + 4 * (g & 1);
+    if (a.splits > 1) {
+      if (m < a.m && col < a.n / 2)
+        *reinterpret_cast<floatx4_t*>(a.part + ((int64_t)split * a.m + m) * a.n + (g < 2 ? 0 : a.n / 2) + col) = acc;
+      return;
+    }
+    float o[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float up = __shfl_xor(acc[r], 32, 64);
+      const float gf = li_to_float(li_from_float<T>(acc[r]));
+      const float s = li_to_float(li_from_float<T>(gf / (1.f + expf(-gf))));
+      o[r] = s * li_to_float(li_from_float<T>(up));
+    }
+    if (g < 2 && m < a.m && col < a.n / 2)
+      *reinterpret_cast<uint2*>(a.out + (m * a.o_s + col) * 2) = uint2{li_pack2<T>(o[0], o[1]), li_pack2<T>(o[2], o[3])};
+  } else {
+    const int col = 16 * group + 4 * g;
+    if (m >= a.m || col >= a.n) return;
+    if (a.splits == 1)
+      *reinterpret_cast<uint2*>(a.out + (m * a.o_s + col) * 2) = uint2{li_pack2<T>(acc[0], acc[1]), li_pack2<T>(acc[2], acc[3])};
+    else
+      *reinterpret_cast<floatx4_t*>(a.part + ((int64_t)split * a.m + m) * a.n + col) = acc;
+  }
+}
 
 // BM: rows of x a work-group holds (m <= BM). R: ring stages.
 template <typename T, int BM, int R, int NW, bool kGate>
@@ -149,39 +226,145 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm(GemmArgs a) {
     __builtin_amdgcn_sched_barrier(0);
   }
 
-  // Lane (m, g): outputs 4g .. 4g + 3 of the wave's 16, row 16 i + m.
 #pragma unroll
-  for (int i = 0; i < kMt; ++i) {
-    const int m = 16 * i + n16;
-    if constexpr (kGate) {
-      // Lanes 0-31 hold gate outputs 0-7, lanes 32-63 the up outputs.
-      const int col = tile * (kTileN / 2) + 8 * w + 4 * (g & 1);
-      float o[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float up = __shfl_xor(acc[i][r], 32, 64);
-        if (a.splits == 1) {
-          const float gf = li_to_float(li_from_float<T>(acc[i][r]));
-          const float s = li_to_float(li_from_float<T>(gf / (1.f + expf(-gf))));
-          o[r] = s * li_to_float(li_from_float<T>(up));
-        }
-      }
-      if (a.splits == 1) {
-        if (g < 2 && m < a.m && col < a.n / 2)
-          *reinterpret_cast<uint2*>(a.out + (m * a.o_s + col) * 2) = uint2{li_pack2<T>(o[0], o[1]), li_pack2<T>(o[2], o[3])};
-      } else if (m < a.m && col < a.n / 2) {
-        *reinterpret_cast<floatx4_t*>(a.part + ((int64_t)split * a.m + m) * a.n + (g < 2 ? 0 : a.n / 2) + col) = acc[i];
-      }
-    } else {
-      const int col = tile * kTileN + 16 * w + 4 * g;
-      if (m >= a.m || col >= a.n) continue;
-      if (a.splits == 1)
-        *reinterpret_cast<uint2*>(a.out + (m * a.o_s + col) * 2) =
-            uint2{li_pack2<T>(acc[i][0], acc[i][1]), li_pack2<T>(acc[i][2], acc[i][3])};
-      else
-        *reinterpret_cast<floatx4_t*>(a.part + ((int64_t)split * a.m + m) * a.n + col) = acc[i];
+  for (int i = 0; i < kMt; ++i) store_outputs<T, kGate>(a, acc[i], split, 16 * i + n16, tile * NW + w, g);
+}
+
+// The same for 65 .. 256 rows, where x is too large to stream beside the
+// weights at their depth: x [BM rows] and W [BN rows] have rings of their own
+// (RX and RW stages of 64 k, rows of 128 bytes, 16-byte chunk c of row r at
+// c ^ (r / 2 % 8): rows two apart share a bank row, so 16 rows' chunks lie in
+// 16 different bank groups). Eight waves, BM / 64 of them along x's rows and
+// the rest along N, each 64 rows by BN / 16 / kWn groups of 16 outputs.
+//
+// Its bound is what a CU loads: 28672 x 4096 at 256 rows takes 71 us with the
+// loads alone (3.1 MB a CU, 44 GB/s; 66 without those of x, 63 without those of
+// W), 55 with the LDS reads and products alone, 78 whole; hence the rule in
+// cut_of.
+template <typename T, int BM, int BN, int RX, int RW, bool kGate>
+__global__ __launch_bounds__(512) void batch_gemm(GemmArgs a) {
+  using M = Mfma<T>;
+  using Frag = typename M::Frag;
+  constexpr int kRow = 128;             // bytes of a row's 64 k
+  constexpr int kWm = BM / 64, kWn = 8 / kWm;
+  constexpr int kNf = BN / 16 / kWn;    // output groups of a wave
+  constexpr int kXi = BM / 64, kWi = BN / 64;  // loads of a wave per stage: eight rows each
+  static_assert(kNf >= 1 && RX == 3 && RW >= 4, "ring depths");
+  __shared__ __attribute__((aligned(1024))) char xring[RX][BM * kRow];
+  __shared__ __attribute__((aligned(1024))) char wring[RW][BN * kRow];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n16 = lane & 15, g = lane >> 4;
+  const int tile = (int)(blockIdx.x / (unsigned)a.splits), split = (int)(blockIdx.x % (unsigned)a.splits);
+  const int total = a.k / 64;
+  const int s0 = (int)((int64_t)total * split / a.splits), s1 = (int)((int64_t)total * (split + 1) / a.splits);
+  const int ns = s1 - s0;
+
+  // Output (weight) row of tile row t.
+  auto weight_row = [&](int t) -> int64_t {
+    if (kGate) {  // of each 16: eight gate rows, then the up rows of the same outputs
+      const int col = min(tile * (BN / 2) + t / 16 * 8 + (t & 7), a.n / 2 - 1);
+      return ((t & 8) ? a.n / 2 : 0) + col;
     }
+    return min(tile * BN + t, a.n - 1);
+  };
+  const int lr = lane >> 3, lc = lane & 7;
+  const char* wrow[kWi];
+  const char* xrow[kXi];
+#pragma unroll
+  for (int i = 0; i < kWi; ++i) {
+    const int t = 8 * (w * kWi + i) + lr;
+    wrow[i] = a.w + weight_row(t) * a.w_s + (int64_t)s0 * kRow + 16 * (lc ^ ((t >> 1) & 7));
   }
+#pragma unroll
+  for (int i = 0; i < kXi; ++i) {
+    const int t = 8 * (w * kXi + i) + lr;
+    xrow[i] = a.x + (int64_t)min(t, a.m - 1) * a.x_s + (int64_t)s0 * kRow + 16 * (lc ^ ((t >> 1) & 7));
+  }
+  const uint32_t xbase = lds_addr(&xring[0][0]), wbase = lds_addr(&wring[0][0]);
+  const unsigned rotated = (unsigned)(tile >> 3) * kRotate;
+  auto at = [&](int st) -> int64_t { return (int64_t)((rotated + (unsigned)st) % (unsigned)ns) * kRow; };
+  auto issue_w = [&](int st) {
+    const uint32_t dst = wbase + (uint32_t)(st % RW) * (BN * kRow) + 1024 * kWi * w;
+    const int64_t o = at(st);
+#pragma unroll
+    for (int i = 0; i < kWi; ++i) dma16<true>(wrow[i] + o, dst + 1024 * i);
+  };
+  auto issue_x = [&](int st) {
+    const uint32_t dst = xbase + (uint32_t)(st % RX) * (BM * kRow) + 1024 * kXi * w;
+    const int64_t o = at(st);
+#pragma unroll
+    for (int i = 0; i < kXi; ++i) dma16<false>(xrow[i] + o, dst + 1024 * i);
+  };
+
+  const int wm = w % kWm, wn = w / kWm;
+  floatx4_t acc[4][kNf];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int f = 0; f < kNf; ++f) acc[i][f] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  uint32_t off[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) off[j] = (uint32_t)(n16 * kRow + 16 * ((4 * j + g) ^ ((n16 >> 1) & 7)));
+
+  Frag w0[kNf], x0[4], w1[kNf] = {}, x1[4] = {};
+  auto read = [&](uint32_t wc, uint32_t xc, int j, Frag (&wf)[kNf], Frag (&xf)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int f = 0; f < kNf; ++f) wf[f] = lds_read_frag<Frag>(wc + f * 16 * kRow + off[j]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) xf[i] = lds_read_frag<Frag>(xc + i * 16 * kRow + off[j]);
+  };
+  auto multiply = [&](const Frag (&wf)[kNf], const Frag (&xf)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int f = 0; f < kNf; ++f) acc[i][f] = M::mma(wf[f], xf[i], acc[i][f]);
+  };
+  auto interleave = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4 + kNf; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // an LDS read
+      __builtin_amdgcn_sched_group_barrier(0x008, (5 * kNf + 3) / (4 + kNf), 0);
+    }
+  };
+
+  // Weights run RW - 1 stages ahead, x two. In order of issue: x 0, x 1 and W
+  // 0 .. RW - 2 first, then x st + 2, W st + RW - 1 in stage st.
+  issue_x(0);
+  if (1 < ns) issue_x(1);
+#pragma unroll
+  for (int st = 0; st < RW - 1; ++st)
+    if (st < ns) issue_w(st);
+  for (int st = 0; st < ns; ++st) {
+    // Loads newer than both W st and x st: in the first two stages those of W
+    // st + 1 .. st + RW - 2 (x 0 and x 1 are older); later W st + RW - 3, x st
+    // + 1 and W st + RW - 2; near the end at least x st + 1.
+    constexpr int kNewer = (RW - 2) * kWi < 2 * kWi + kXi ? (RW - 2) * kWi : 2 * kWi + kXi;
+    if (st + RW - 1 < ns) li_wait_vm<kNewer>();
+    else if (st >= 2 && st + 1 < ns) li_wait_vm<kXi>();
+    else li_wait_vm<0>();
+    lds_barrier();
+    if (st + 2 < ns) issue_x(st + 2);
+    if (st + RW - 1 < ns) issue_w(st + RW - 1);
+    const uint32_t xc = xbase + (uint32_t)(st % RX) * (BM * kRow) + (uint32_t)wm * 64 * kRow;
+    const uint32_t wc = wbase + (uint32_t)(st % RW) * (BN * kRow) + (uint32_t)wn * kNf * 16 * kRow;
+    // A half stage's operands are read while the half before is multiplied
+    // (across the barrier: the second half of stage st - 1 under the reads of
+    // the first half of st), one read with every few products.
+    read(wc, xc, 0, w0, x0);
+    multiply(w1, x1);
+    interleave();
+    read(wc, xc, 1, w1, x1);
+    multiply(w0, x0);
+    interleave();
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  multiply(w1, x1);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int f = 0; f < kNf; ++f)
+      store_outputs<T, kGate>(a, acc[i][f], split, 64 * wm + 16 * i + n16, tile * (BN / 16) + wn * kNf + f, g);
 }
 
 // out = the sum of the splits' fp32 sums, rounded.
@@ -206,17 +389,29 @@ __global__ __launch_bounds__(256) void skinny_reduce(const float* part, char* ou
 }
 
 template <typename T, int BM, int R, int NW>
-void launch(const GemmArgs& a, hipStream_t s) {
+void launch_skinny(const GemmArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)((a.n + 16 * NW - 1) / (16 * NW) * a.splits)), block(64 * NW);
   if (a.gate) hipLaunchKernelGGL((skinny_gemm<T, BM, R, NW, true>), grid, block, 0, s, a);
   else hipLaunchKernelGGL((skinny_gemm<T, BM, R, NW, false>), grid, block, 0, s, a);
 }
 
+template <typename T, int BM, int BN, int RW>
+void launch_batch(const GemmArgs& a, hipStream_t s) {
+  const dim3 grid((unsigned)((a.n + BN - 1) / BN * a.splits)), block(512);
+  if (a.gate) hipLaunchKernelGGL((batch_gemm<T, BM, BN, 3, RW, true>), grid, block, 0, s, a);
+  else hipLaunchKernelGGL((batch_gemm<T, BM, BN, 3, RW, false>), grid, block, 0, s, a);
+}
+
 template <typename T>
 void launch_rows(const GemmArgs& a, hipStream_t s) {
-  if (a.m <= 16) launch<T, 16, 4, 4>(a, s);
-  else if (a.m <= kFewRows) launch<T, 32, 3, 4>(a, s);
-  else launch<T, 64, 3, 8>(a, s);
+  const bool wide = cut_of(a.m, a.n, a.k).tile == 128;
+  if (a.m <= 16) launch_skinny<T, 16, 4, 4>(a, s);
+  else if (a.m <= kFewRows) launch_skinny<T, 32, 3, 4>(a, s);
+  else if (a.m <= kSkinnyRows) launch_skinny<T, 64, 3, 8>(a, s);
+  else if (a.m <= 128 && wide) launch_batch<T, 128, 128, 6>(a, s);
+  else if (a.m <= 128) launch_batch<T, 128, 64, 8>(a, s);
+  else if (wide) launch_batch<T, 256, 128, 4>(a, s);
+  else launch_batch<T, 256, 64, 6>(a, s);
 }
 
 }  // namespace
@@ -227,13 +422,10 @@ extern "C" int li_skinny_gemm_plan(int m, int n, int k, int* splits) {
   if (m > LI_SKINNY_MAX_ROWS || n % 8 || k % kStageK)
     return li::fail(LI_EUNSUPPORTED, "li_skinny_gemm: up to %d rows, n a multiple of 8, k of %d; got %d, %d, %d",
                     LI_SKINNY_MAX_ROWS, kStageK, m, n, k);
-  // As many runs of K as fill the GPU once, at least one stage each; none
-  // where the tiles alone are three quarters of a work-group a CU or more
-  // (what a second run gains is less than adding the sums costs: 16,032 x
-  // 4,096 at 8 rows 21.5 us whole, 26.9 in two, 21.4 in four).
-  const int tiles = (n + tile_of(m) - 1) / tile_of(m), cus = li::device_cu_count();
-  const int want = tiles * 4 >= cus * 3 ? 1 : cus * per_cu(m) / tiles;
-  if (splits) *splits = std::max(1, std::min(want, k / kStageK));
+  const Cut cut = cut_of(m, n, k);
+  if (cut.splits == 0)
+    return li::fail(LI_EUNSUPPORTED, "li_skinny_gemm: %d rows of %d x %d are a general GEMM's", m, n, k);
+  if (splits) *splits = cut.splits;
   return LI_OK;
 }
 

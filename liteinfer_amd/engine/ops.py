@@ -35,9 +35,10 @@ class Partials(NamedTuple):
     """The projection's shape, ``[..., n]``."""
 
 
-# Rows of x up to which the projections run as this library's kernel
-# (LI_SKINNY_MAX_ROWS); torch's GEMMs serve larger passes.
-SKINNY_MAX_ROWS = 64
+# Rows of x up to which the projections may run as this library's kernels
+# (LI_SKINNY_MAX_ROWS; li_skinny_gemm_plan says which); torch's GEMMs serve
+# the others.
+SKINNY_MAX_ROWS = 256
 
 
 @functools.lru_cache(maxsize=4096)
@@ -46,7 +47,10 @@ def _splits(rows: int, n: int, k: int) -> int:
     if rows > SKINNY_MAX_ROWS or n % 8 or k % 128:
         return 0
     splits = ctypes.c_int()
-    _native.check(_native.load().li_skinny_gemm_plan(rows, n, k, ctypes.byref(splits)), "skinny_gemm")
+    status = _native.load().li_skinny_gemm_plan(rows, n, k, ctypes.byref(splits))
+    if status == _native.LI_EUNSUPPORTED:
+        return 0
+    _native.check(status, "skinny_gemm")
     return splits.value
 
 

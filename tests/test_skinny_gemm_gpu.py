@@ -1,7 +1,7 @@
 """The decode step's projections (engine/ops.py: linear, linear_sums, gate_up_silu) against float64 products.
 
-Sizes at the kernel's edges: one row, the row blocks of 16 / 32 / 64 and one
-past them, weight rows that fill no 128-row tile, one 128-k stage, and K cut
+Sizes at the kernel's edges: one row, the row blocks of 16 / 32 / 64 / 128 / 256
+and one past them, weight rows that fill no 128-row tile, one 128-k stage, and K cut
 into many runs. Bound: the product of N(0, 1) x and 0.02 N(0, 1) w in fp32,
 rounded once: half an ulp (at most 2^-8 relative in bf16, 2^-11 in fp16) plus fp32
 summation error, well under 1e-4 here.
@@ -33,18 +33,20 @@ def _close(got, want, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("rows", [1, 2, 15, 16, 17, 32, 33, 64])
-@pytest.mark.parametrize("n,k", [(128, 128), (120, 256), (1000, 1152), (6144, 4096), (256, 14336), (33000, 256)])
+@pytest.mark.parametrize("rows", [1, 2, 15, 16, 17, 32, 33, 64, 65, 128, 129, 256])
+@pytest.mark.parametrize("n,k", [(128, 128), (120, 256), (1000, 1152), (6144, 4096), (4088, 4096), (256, 14336), (33000, 256)])
 def test_linear(rows, n, k, dtype):
     x, w, want = _inputs(rows, n, k, dtype)
-    assert ops._skinny(x, w)[1] > 0
+    splits = ops._skinny(x, w)[1]
+    if rows <= 64 or (n, k) == (6144, 4096) or (n, k, rows) in ((4088, 4096, 65), (4088, 4096, 129), (33000, 256, 128)):
+        assert splits > 0  # (whole tiles, and runs in 128- and 64-row tiles, past 64 rows)
     _close(ops.linear(x, w), want, dtype)
     sums = ops.linear_sums(x, w)
     if isinstance(sums, ops.Partials):
         assert (sums.sums.double().sum(0) - want).abs().max() < 1e-4
 
 
-@pytest.mark.parametrize("rows", [1, 16, 24, 64])
+@pytest.mark.parametrize("rows", [1, 16, 24, 64, 100, 200])
 @pytest.mark.parametrize("ffn", [64, 1032, 14336])
 def test_gate_up(rows, ffn):
     x, w, want = _inputs(rows, 2 * ffn, 512, torch.bfloat16)
@@ -75,7 +77,7 @@ def test_norm_adds_the_runs(rows, splits):
 
 
 def test_rows_it_does_not_serve_run_as_torch_products():
-    x, w, want = _inputs(65, 256, 256, torch.bfloat16)
+    x, w, want = _inputs(257, 256, 256, torch.bfloat16)
     assert ops._skinny(x, w)[1] == 0
     _close(ops.linear(x, w), want, torch.bfloat16)
     x, w, want = _inputs(4, 256, 192, torch.bfloat16)
