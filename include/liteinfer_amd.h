@@ -445,6 +445,29 @@ int li_silu_mul_partials(const float* partials, int splits, void* out,
                          int64_t rows, int ffn, int64_t out_stride, int dtype,
                          void* stream);
 
+/*
+ * The engine's per-step inputs, one launch each (chains of torch copies and
+ * elementwise ops otherwise).
+ *
+ * li_rotary_tables: cos / sin [tokens, 2 half] of dtype, of positions[t] *
+ * inv_freq[d mod half] in fp32 (liteinfer/models/llama.py:70-78).
+ * li_stage_decode: a decode step's token ids, positions, write slots, context
+ * lengths (n each) and slot table ([n, cols], row stride slots_stride) into
+ * the static buffers of a captured step of `width` rows (table rows
+ * table_stride apart); rows n .. width - 1 become a one-token context in
+ * pad_slot (liteinfer/engine/cuda_graphs.py).
+ */
+int li_rotary_tables(const int64_t* positions, const float* inv_freq,
+                     void* cos_out, void* sin_out, int64_t tokens, int half,
+                     int dtype, void* stream);
+int li_stage_decode(const int64_t* ids, const int64_t* positions,
+                    const int64_t* write_slots, const int64_t* slots,
+                    int64_t slots_stride, const int32_t* context_lens,
+                    int64_t* ids_out, int64_t* positions_out,
+                    int64_t* write_out, int64_t* table_out,
+                    int64_t table_stride, int32_t* lens_out, int n, int cols,
+                    int width, int64_t pad_slot, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -59,6 +59,8 @@ EXPORTED_SYMBOLS = (
     "li_skinny_reduce",
     "li_add_rms_norm_partials",
     "li_silu_mul_partials",
+    "li_rotary_tables",
+    "li_stage_decode",
 )
 
 _i64, _i32, _p, _f32, _sz = ctypes.c_int64, ctypes.c_int, ctypes.c_void_p, ctypes.c_float, ctypes.c_size_t
@@ -72,6 +74,8 @@ _SIGNATURES = {
     "li_skinny_reduce": (_i32, [_p, _p, _i64, _i32, _i32, _i32, _i32, _p]),
     "li_add_rms_norm_partials": (_i32, [_p, _p, _i32, _p, _p, _i64, _i32, _i64, _i64, _f32, _i32, _p]),
     "li_silu_mul_partials": (_i32, [_p, _i32, _p, _i64, _i32, _i64, _i32, _p]),
+    "li_rotary_tables": (_i32, [_p, _p, _p, _p, _i64, _i32, _i32, _p]),
+    "li_stage_decode": (_i32, [_p, _p, _p, _p, _i64, _p, _p, _p, _p, _p, _i64, _p, _i32, _i32, _i32, _i64, _p]),
     "li_last_error_string": (ctypes.c_char_p, []),
     "li_abi_version": (_i32, []),
     "li_build_id": (ctypes.c_char_p, []),

@@ -105,6 +105,8 @@ class RandomLlama:
 
     def _rotary(self, positions: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         """cos / sin ``[B, T, D]`` in the model dtype, computed in fp32 (llama.py:70-78)."""
+        if self._fused_ops:
+            return self._fused_ops.rotary_tables(positions, self.inv_freq, self.dtype)
         freqs = positions[..., None].to(torch.float32) * self.inv_freq
         emb = torch.cat((freqs, freqs), dim=-1)
         return emb.cos().to(self.dtype), emb.sin().to(self.dtype)

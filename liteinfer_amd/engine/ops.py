@@ -1,4 +1,6 @@
-"""The minimal engine's fused elementwise ops on a ROCm device (`li_add_rms_norm`, `li_silu_mul`).
+"""The minimal engine's own ops on a ROCm device: fused elementwise work (`li_add_rms_norm`,
+`li_silu_mul`), the decode step's projections (`li_skinny_gemm`) and its inputs (`li_rotary_tables`,
+`li_stage_decode`).
 
 Same results as the model's torch ops (liteinfer/models/llama.py:34-48,
 :101-116) up to the order of the fp32 sum of squares and the exponential's
@@ -156,3 +158,40 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
                                         _native.dtype_code(gate_up.dtype), _native.stream_handle(gate_up.device))
     _native.check(status, "silu_mul")
     return out
+
+
+def rotary_tables(positions: torch.Tensor, inv_freq: torch.Tensor, dtype: torch.dtype) -> tuple[torch.Tensor, torch.Tensor]:
+    """cos / sin ``[..., D]`` of `positions` times `inv_freq` (``[D / 2]`` fp32, each twice), rounded to `dtype`."""
+    positions = positions.to(torch.int64).contiguous()
+    half = inv_freq.shape[0]
+    cos, sin = (torch.empty(*positions.shape, 2 * half, dtype=dtype, device=positions.device) for _ in range(2))
+    status = _native.load().li_rotary_tables(
+        positions.data_ptr(), inv_freq.data_ptr(), cos.data_ptr(), sin.data_ptr(), positions.numel(), half,
+        _native.dtype_code(dtype), _native.stream_handle(positions.device))
+    _native.check(status, "rotary_tables")
+    return cos, sin
+
+
+def stage_decode(inputs: tuple[torch.Tensor, ...], static: tuple[torch.Tensor, ...], width: int, pad_slot: int) -> None:
+    """A decode step's (ids, positions, write slots, slot table, context lengths) into a captured graph's buffers.
+
+    `static` holds the buffers in the same order; rows past the step's, up to
+    `width`, become a one-token context in `pad_slot`.
+    """
+    ids, positions, write_slots, slots, lens = inputs
+    n, cols = slots.shape
+    device = static[0].device
+
+    def column(t: torch.Tensor, shape: tuple[int, ...], dtype: torch.dtype) -> torch.Tensor:
+        return torch.broadcast_to(t, shape).to(device=device, dtype=dtype).contiguous()
+
+    ids, positions = column(ids, (n, 1), torch.int64), column(positions, (n, 1), torch.int64)
+    write_slots, lens = column(write_slots, (1, n), torch.int64), column(lens, (n,), torch.int32)
+    slots = slots.to(device=device, dtype=torch.int64)
+    if slots.stride(-1) != 1:
+        slots = slots.contiguous()
+    status = _native.load().li_stage_decode(
+        ids.data_ptr(), positions.data_ptr(), write_slots.data_ptr(), slots.data_ptr(), slots.stride(0), lens.data_ptr(),
+        static[0].data_ptr(), static[1].data_ptr(), static[2].data_ptr(), static[3].data_ptr(), static[3].stride(0),
+        static[4].data_ptr(), n, cols, width, pad_slot, _native.stream_handle(device))
+    _native.check(status, "stage_decode")

@@ -20,6 +20,7 @@ import torch
 from liteinfer_amd.cache.block_pool import to_device
 from liteinfer_amd.cache.kv_cache import KVCache
 from liteinfer_amd.engine.model import RandomLlama
+from liteinfer_amd.engine.ops import stage_decode
 from liteinfer_amd.engine.scheduler import PENDING_TOKEN, Sequence
 
 _PAD = "__pad__"
@@ -121,17 +122,12 @@ class DecodeGraphs:
     def run(self, input_ids, positions, write_slots, slots, context_lens) -> torch.Tensor:
         n, cols = slots.shape
         width = self._width_for(n)
-        self.input_ids[:n].copy_(input_ids)
-        self.positions[:n].copy_(positions)
-        self.write_slots[:, :n].copy_(write_slots)
-        self.slot_table[:n, :cols].copy_(slots)
-        self.context_lens[:n].copy_(context_lens)
-        if n < width:  # padding rows: one key in the reserved slot
-            self.input_ids[n:width].zero_()
-            self.positions[n:width].zero_()
-            self.write_slots[:, n:width].fill_(self.pad_slot)
-            self.slot_table[n:width, 0].fill_(self.pad_slot)
-            self.context_lens[n:width].fill_(1)
+        if n > self.slot_table.shape[0] or cols > self.slot_table.shape[1]:
+            raise ValueError(f"a step of {n} x {cols} slots does not fit the captured "
+                             f"{tuple(self.slot_table.shape)} table")
+        stage_decode((input_ids, positions, write_slots, slots, context_lens),
+                     (self.input_ids, self.positions, self.write_slots, self.slot_table, self.context_lens),
+                     width, self.pad_slot)
         if width not in self._graphs:
             self._capture(width)
         graph, out = self._graphs[width]
