@@ -68,7 +68,9 @@ struct Cut {
 
 // Up to 64 rows every projection measured faster here than through hipBLASLt
 // (1.0 .. 3.0 times, 10 shapes of the 8B and 1B architectures). K is cut into
-// as many runs as fill the GPU once, at least one stage each; not at all where
+// as many runs as fill the GPU once, of at least two stages (of one, the sums
+// cost the norm more than the run saves: a step of 4 layers of the 1B
+// architecture at 24 rows 322 -> 312 us); not at all where
 // the tiles alone are three quarters of a work-group a CU or more (what a
 // second run gains is less than adding the sums costs: 16,032 x 4,096 at 8
 // rows 21.5 us whole, 26.9 in two).
@@ -92,7 +94,7 @@ Cut cut_of(int m, int n, int k) {
   auto tiles = [&](int tile) { return (n + tile - 1) / tile; };
   auto runs = [&](int tile, int per_cu) {
     const int t = tiles(tile);
-    return t * 4 >= cus * 3 ? 1 : std::max(1, std::min(cus * per_cu / t, stages));
+    return t * 4 >= cus * 3 ? 1 : std::max(1, std::min(cus * per_cu / t, stages / 2));
   };
   if (m <= kFewRows) return {64, runs(64, 2)};  // (two work-groups a CU)
   if (m <= kSkinnyRows) return {128, runs(128, 1)};
