@@ -24,6 +24,7 @@ PACKAGE_DIR = Path(__file__).resolve().parent
 CSRC_DIR = PACKAGE_DIR / "csrc"
 LIB_DIR = PACKAGE_DIR / "_lib"
 LIB_PATH = LIB_DIR / "libliteinfer_amd.so"
+FAST_CALLS_PATH = LIB_DIR / "_fast_calls.so"
 INCLUDE_DIR = PACKAGE_DIR.parent / "include"
 
 OFFLOAD_ARCH = "gfx950"
@@ -95,14 +96,35 @@ def _compile(src: Path, obj: Path, build_id: str) -> None:
         print(err, file=sys.stderr)
 
 
+def _compile_fast_calls(build_id: str) -> None:
+    """csrc/fast_calls.cpp, the eager calls' host side: a Python extension against this interpreter's torch."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    torch_lib = Path(torch.__file__).resolve().parent / "lib"
+    out_tmp = LIB_DIR / (FAST_CALLS_PATH.name + ".tmp")
+    cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-w",
+           f'-DLI_BUILD_ID="{build_id}"', f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-I{p}" for p in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"])),
+           str(CSRC_DIR / "fast_calls.cpp"), "-o", str(out_tmp),
+           f"-L{torch_lib}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed on fast_calls.cpp:\n{proc.stderr}")
+    os.replace(out_tmp, FAST_CALLS_PATH)
+
+
 def build(verbose: bool = False) -> Path:
-    """Compile every source and link the library. Always rebuilds."""
+    """Compile every source and link the libraries. Always rebuilds."""
     LIB_DIR.mkdir(parents=True, exist_ok=True)
     build_id = source_hash()
     with tempfile.TemporaryDirectory(prefix="liteinfer_amd_build_") as tmp:
         objs = []
         jobs = []
         with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as pool:
+            jobs.append(pool.submit(_compile_fast_calls, build_id))
             for src in sources():
                 obj = Path(tmp) / (src.stem + ".o")
                 objs.append(obj)

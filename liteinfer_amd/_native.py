@@ -9,6 +9,8 @@ the paged path refuses to run and says how to build it.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import threading
 from pathlib import Path
 
@@ -186,6 +188,37 @@ def load() -> ctypes.CDLL:
                 )
             _lib = lib
     return _lib
+
+
+_fast = None
+
+
+def fast_calls():
+    """The eager calls' host side in C++ (``csrc/fast_calls.cpp``), bound to the loaded library.
+
+    Its functions return None for every call they leave to the Python code.
+    """
+    global _fast
+    if _fast is not None:
+        return _fast
+    lib = load()
+    with _lock:
+        if _fast is None:
+            path = _build.FAST_CALLS_PATH
+            if not path.exists():
+                raise NativeLibraryMissing(f"{path} is missing; run `python -m liteinfer_amd._build`")
+            loader = importlib.machinery.ExtensionFileLoader("_fast_calls", str(path))
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_fast_calls", loader))
+            loader.exec_module(module)
+            expected = _build.source_hash()
+            if module.build_id != expected:
+                raise RuntimeError(f"{path} was built from other sources (build id {module.build_id}, the sources here "
+                                   f"hash to {expected}); rebuild it with `python -m liteinfer_amd._build`")
+            module.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in (
+                "li_paged_decode_plan", "li_paged_decode_write", "li_paged_prefill_plan", "li_paged_prefill_ex",
+                "li_rope_kv_write", "li_rope_kv_write_fp8")))
+            _fast = module
+    return _fast
 
 
 def last_error() -> str:

@@ -50,12 +50,13 @@ _MAX_SPLITS = 32
 _MI355X_COMPUTE_UNITS = 256
 
 _KERNELS = ("auto", "generic", "equal_splits")
+_FLAGS = {"auto": 0, "generic": _native.LI_FLAG_FORCE_GENERIC, "equal_splits": _native.LI_FLAG_EQUAL_SPLITS}
 
 
 def _flags(kernel: str) -> int:
     if kernel not in _KERNELS:
         raise ValueError(f"kernel must be one of {_KERNELS}, got {kernel!r}")
-    return {"auto": 0, "generic": _native.LI_FLAG_FORCE_GENERIC, "equal_splits": _native.LI_FLAG_EQUAL_SPLITS}[kernel]
+    return _FLAGS[kernel]
 
 
 def _prefill_kernel(kernel: str) -> str:
@@ -351,6 +352,15 @@ def paged_decode(
     Returns:
         ``[batch, num_heads, head_dim]``, same dtype as ``query``.
     """
+    if query.is_cuda and kernel in _FLAGS and (num_splits is None or num_splits > 0):
+        # Operands that need no conversion: checked and passed on in C++.
+        out = _native.fast_calls().decode(
+            query, key_pool, value_pool, slot_table, context_lens, scaling, num_kv_groups, block_kv, num_splits or 0,
+            _FLAGS[kernel], k_scale, v_scale, new_key, new_value, _native.stream_handle(query.device))
+        if out is not None:
+            if isinstance(out, int):
+                _native.check(out, "paged_decode")
+            return out
     device, query, slot_table, context_lens, kv_code = _decode_inputs(
         query, key_pool, value_pool, slot_table, context_lens, num_kv_groups, num_splits, k_scale, v_scale)
     batch, num_heads, head_dim = query.shape
@@ -499,6 +509,16 @@ def paged_prefill(
         ``[total_queries, num_heads, head_dim]`` (`out`, or a new tensor with
         the strides of `query`).
     """
+    if query.is_cuda and kernel in ("auto", "generic"):
+        # Operands that need no conversion: checked and passed on in C++.
+        flags = _FLAGS[kernel] | (_native.LI_FLAG_PREFILL_ONLY if one_query_rows is False else 0)
+        got = _native.fast_calls().prefill(
+            query, key_pool, value_pool, slot_table, context_lens, query_start_loc, max_query_len, scaling,
+            num_kv_groups, block_kv, block_q, flags, k_scale, v_scale, out, _native.stream_handle(query.device))
+        if got is not None:
+            if isinstance(got, int):
+                _native.check(got, "paged_prefill")
+            return got
     if key_pool.stride() != value_pool.stride():
         raise ValueError("key and value pools must be laid out identically")
     device = _require_device_tensors(query, key_pool, value_pool, slot_table, context_lens, query_start_loc)

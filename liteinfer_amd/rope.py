@@ -69,6 +69,14 @@ def rope_kv_write(
         token-major in memory like the reference's result (so the packed
         attention's ``squeeze(0).transpose(0, 1)`` is a free view).
     """
+    if q.is_cuda:
+        # Operands that need no conversion: checked and passed on in C++.
+        out = _native.fast_calls().rope(q, k, v, cos, sin, slots, key_pool, value_pool, k_scale, v_scale, bad_slots,
+                                        _native.stream_handle(q.device))
+        if out is not None:
+            if isinstance(out, int):
+                _native.check(out, "rope_kv_write")
+            return out
     device = _require_device_tensors(q, k, v, cos, sin, slots, key_pool, value_pool)
     bad_ptr = bad_slots_pointer(bad_slots, device)
     _check_pools(key_pool, value_pool)
