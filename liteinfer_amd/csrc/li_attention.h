@@ -193,9 +193,10 @@ int launch_decode_mfma(const AttnArgs& a, int dtype, hipStream_t s);
 constexpr int kShortChunk = 256;
 // Sequences of a packed pass the direct prefill schedule serves (a pass
 // whose every unit has a work-group of its own, no one-query rows in the
-// launch, no split: no work list; work-group i takes
-// unit i / (queue count) of its queue, found by one wave's scan of the
-// sequences' query counts, and nothing after it).
+// launch: no work list; work-group i takes unit i / (queue count) of its
+// queue, found by one wave's scan of the sequences' query counts, and nothing
+// after it. A split pass's units are its pieces; those of head_dim 128 keep
+// the list).
 constexpr int kPrefillDirectBatch = 64;
 // Its rule: segments (sequence, KV head) x max_context at most
 // kShortMaxKeySegments, and max_context at most kShortMaxWidth, or twice that

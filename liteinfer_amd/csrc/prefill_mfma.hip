@@ -199,6 +199,94 @@ __device__ __forceinline__ int4 direct_entry(const AttnArgs& a, int want) {
   return int4{sq * a.num_qblocks + qb, __shfl(e.x, sq, 64), __shfl(e.y, sq, 64), __shfl(e.z, sq, 64)};
 }
 
+// A pass too small to fill the grid is cut into pieces (AttnArgs::split_ok):
+// each block's fully visible stages -- wholly before its first query -- into
+// up to f pieces of at least kSplitMinStages stages, f the grid's units over
+// the blocks' units. The last piece also takes the stages its queries mask,
+// so every piece's every row sees a key. A block's pieces are consecutive
+// entries, a sequence's blocks last first, in sequence order.
+__device__ __forceinline__ int split_limit(const AttnArgs& a, int blocks) {
+  return max(1, a.split_target / max(1, blocks * a.num_kv_heads));
+}
+// Block qb of a sequence of nq queries and ctx keys: its stages, the fully
+// visible ones and its pieces.
+__device__ __forceinline__ int split_cut(const AttnArgs& a, int f, int nq, int ctx, int qb, int* ns, int* vis) {
+  const int bq = a.block_q;
+  const int nblk = (nq + bq - 1) / bq;
+  const int q1 = nq - (nblk - 1 - qb) * bq;
+  const int q0 = max(q1 - bq, 0);
+  const int pos0 = ctx - nq;
+  *ns = (pos0 + q1 + kStageKeys - 1) / kStageKeys;
+  *vis = (pos0 + q0 + 1) / kStageKeys;
+  return max(1, min(min(f, kSplitMaxPieces), *vis / kSplitMinStages));
+}
+__device__ __forceinline__ int4 split_range(int k, int p, int ns, int vis) {
+  const int per = vis / p;
+  return int4{k * per, k + 1 < p ? (k + 1) * per : ns, k, p};
+}
+
+// The direct schedule of a split pass (no work list; at most 64 sequences,
+// none served elsewhere): one full wave finds, from the sequences' query
+// counts, entry `want` of the list prefill_order would write and its stage
+// range, or with kBlock the want-th block of several pieces (then `at` is its
+// first entry). {-1, 0, 0, 0} past the last. Every lane returns it. The scan
+// is a handful of loads and shuffles; the list is a launch of one work-group
+// that everything waits for (both measured at the launch).
+template <bool kBlock>
+__device__ __forceinline__ int4 direct_split_entry(const AttnArgs& a, int want, int4& range, int& at) {
+  const int lane = (int)(threadIdx.x & 63);
+  int first = 0, nq = 0, ctx = 0, nb = 0;
+  if (lane < a.batch) {
+    first = a.qsl[lane];
+    nq = a.qsl[lane + 1] - first;
+    ctx = a.ctx[lane];
+    if (nq > 0) nb = min((nq + a.block_q - 1) / a.block_q, a.num_qblocks);
+  }
+  int blocks = nb;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) blocks += __shfl_xor(blocks, off, 64);
+  const int f = split_limit(a, blocks);
+  int entries = 0, cuts = 0;  // of this lane's sequence
+  for (int i = 0; i < nb; ++i) {
+    int ns, vis;
+    const int p = split_cut(a, f, nq, ctx, nb - 1 - i, &ns, &vis);
+    entries += p;
+    cuts += p > 1;
+  }
+  int e_incl = entries, c_incl = cuts;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int e_up = __shfl_up(e_incl, off, 64), c_up = __shfl_up(c_incl, off, 64);
+    if (lane >= off) {
+      e_incl += e_up;
+      c_incl += c_up;
+    }
+  }
+  const uint64_t hit = __ballot((kBlock ? c_incl : e_incl) > want);
+  range = int4{0, 0x7fffffff, 0, 1};
+  at = 0;
+  if (hit == 0) return int4{-1, 0, 0, 0};
+  const int sq = __ffsll((long long)hit) - 1;
+  first = __shfl(first, sq, 64);
+  nq = __shfl(nq, sq, 64);
+  ctx = __shfl(ctx, sq, 64);
+  nb = __shfl(nb, sq, 64);
+  at = __shfl(e_incl - entries, sq, 64);
+  int left = want - (kBlock ? __shfl(c_incl - cuts, sq, 64) : at);
+  for (int i = 0; i < nb; ++i) {
+    int ns, vis;
+    const int qb = nb - 1 - i, p = split_cut(a, f, nq, ctx, qb, &ns, &vis);
+    const int mine = kBlock ? p > 1 : p;
+    if (left < mine) {
+      range = split_range(kBlock ? 0 : left, p, ns, vis);
+      return int4{sq * a.num_qblocks + qb, first, nq, ctx};
+    }
+    left -= mine;
+    at += p;
+  }
+  return int4{-1, 0, 0, 0};
+}
+
 // Keys whose slots the lockstep kernel stages in LDS at a time (restaging
 // costs a pipeline drain, so chunks are long).
 constexpr int kLockstepChunk = 4096;
@@ -741,14 +829,17 @@ __device__ __forceinline__ void prefill_pp_body(AttnArgs a, const AttnArgs& d) {
   };
   if constexpr (kDirect) {
     // Unit wg / nqueues of this queue: entry (wg / nqueues) / heads_per_queue
-    // of the blocks prefill_order would list (direct_entry).
+    // of those prefill_order would list (direct_entry, direct_split_entry).
     if (tid < 64) {
       const int u = (int)(wg / (unsigned)nqueues);
-      const int4 e = direct_entry(a, u / heads_per_queue);
+      int4 e, r{};
+      int first_entry;
+      if constexpr (kSplit) e = direct_split_entry<false>(a, u / heads_per_queue, r, first_entry);
+      else e = direct_entry(a, u / heads_per_queue);
       if (lane == 0) {
         s_unit = e.x < 0 ? kNoUnit : u;
         s_entry = e;
-        if constexpr (kSplit) s_range = int4{0, 0x7fffffff, 0, 1};
+        if constexpr (kSplit) s_range = r;
       }
     }
   } else if (tid == 0) {
@@ -1085,7 +1176,7 @@ __device__ __forceinline__ void prefill_pp_body(AttnArgs a, const AttnArgs& d) {
     // load, where the compiler places its wait for the atomic (this file is
     // built with the wave-level atomic optimizer off, which would otherwise
     // read the value back at once and wait for every load in flight).
-    if (j == claim_at && tid == 0) next_unit = kDirect ? kNoUnit : atomicAdd(&a.queue[qi], 1);
+    if (!kDirect && j == claim_at && tid == 0) next_unit = atomicAdd(&a.queue[qi], 1);
     if (!idle) {
       // The matrix phase issues ahead of the other wave's vector work on
       // its SIMD: an MFMA that waits for issue leaves the matrix core idle.
@@ -1148,7 +1239,7 @@ __device__ __forceinline__ void prefill_pp_body(AttnArgs a, const AttnArgs& d) {
   // tid 0 reads the next unit's work-list entry (its id came back from the
   // claim above) while the last P V runs.
   int4 next_entry{-1, 0, 0, 0}, next_range{0, 0x7fffffff, 0, 1};
-  if (tid == 0) {
+  if (!kDirect && tid == 0) {
     next_entry = entry_of(next_unit);
     if constexpr (kSplit) next_range = range_of(next_unit);
   }
@@ -1159,13 +1250,13 @@ __device__ __forceinline__ void prefill_pp_body(AttnArgs a, const AttnArgs& d) {
   }
   lds_barrier();
   if (!late) lds_barrier();  // the barrier waves 4-7 took first
-  if (tid == 0) {
+  if (!kDirect && tid == 0) {
     s_unit = next_unit;
     s_entry = next_entry;
     if constexpr (kSplit) s_range = next_range;
   }
   lds_barrier();
-  {
+  if constexpr (!kDirect) {
     // The next unit's first slots, read now so that their round trip runs
     // under this unit's output stores.
     const int nu = __builtin_amdgcn_readfirstlane(s_unit);
@@ -1194,6 +1285,7 @@ __device__ __forceinline__ void prefill_pp_body(AttnArgs a, const AttnArgs& d) {
           *reinterpret_cast<float2*>(a.split_ml + (slot * kMinRows + r) * 2) = float2{m[nb], acc[nb][kBlk][0]};
       }
     }
+    if (kDirect) break;  // (its one unit)
     continue;
   }
   // The output rows, normalised. A lane holds 8-byte pieces of its row 32
@@ -1248,6 +1340,7 @@ __device__ __forceinline__ void prefill_pp_body(AttnArgs a, const AttnArgs& d) {
       }
     }
   }
+  if (kDirect) break;
   }  // units
 }
 
@@ -1312,12 +1405,8 @@ __global__ __launch_bounds__(1024) void prefill_order(AttnArgs a) {
   const bool has_rows = __syncthreads_or(tid < a.batch && c_e.y == 1 && a.single_query_elsewhere);
   if (a.split_ok && !has_rows) {
     // A pass too small to fill the grid (the host allows this only for a
-    // batch of at most 1024 sequences, so thread i holds sequence i): each
-    // block's fully visible stages -- wholly before its first query -- are
-    // cut into up to f pieces of at least kSplitMinStages stages, f the
-    // grid's units over the blocks' units. The last piece also takes the
-    // stages its queries mask, so every piece's every row sees a key. A
-    // block's pieces are consecutive entries, in sequence order.
+    // batch of at most 1024 sequences, so thread i holds sequence i): the
+    // blocks are cut into pieces (split_cut).
     __shared__ int s_blocks, s_split;
     __shared__ int s_wave[1024 / 64];
     if (tid == 0) {
@@ -1327,19 +1416,8 @@ __global__ __launch_bounds__(1024) void prefill_order(AttnArgs a) {
     __syncthreads();
     if (c_nb > 0) atomicAdd(&s_blocks, c_nb);
     __syncthreads();
-    const int f = max(1, a.split_target / max(1, s_blocks * a.num_kv_heads));
-    const int bq = a.block_q;
-    // Block qb of this thread's sequence: its stage count and its pieces.
-    auto cut = [&](int qb, int* ns, int* vis) -> int {
-      const int nq = c_e.y, ctx = c_e.z;
-      const int nblk = (nq + bq - 1) / bq;
-      const int q1 = nq - (nblk - 1 - qb) * bq;
-      const int q0 = max(q1 - bq, 0);
-      const int pos0 = ctx - nq;
-      *ns = (pos0 + q1 + kStageKeys - 1) / kStageKeys;
-      *vis = (pos0 + q0 + 1) / kStageKeys;
-      return max(1, min(min(f, kSplitMaxPieces), *vis / kSplitMinStages));
-    };
+    const int f = split_limit(a, s_blocks);
+    auto cut = [&](int qb, int* ns, int* vis) -> int { return split_cut(a, f, c_e.y, c_e.z, qb, ns, vis); };
     int mine = 0;
     for (int i = 0; i < c_nb; ++i) {
       int ns, vis;
@@ -1361,11 +1439,10 @@ __global__ __launch_bounds__(1024) void prefill_order(AttnArgs a) {
       const int qb = c_nb - 1 - i;
       int ns, vis;
       const int p = cut(qb, &ns, &vis);
-      const int per = vis / p;
       if (p > 1) a.split_first[atomicAdd(&s_split, 1)] = at;
       for (int k = 0; k < p; ++k, ++at) {
         a.work[at] = int4{tid * a.num_qblocks + qb, c_e.x, c_e.y, c_e.z};
-        a.work_range[at] = int4{k * per, k + 1 < p ? (k + 1) * per : ns, k, p};
+        a.work_range[at] = split_range(k, p, ns, vis);
       }
     }
     if (tid < kPrefillQueues) a.queue[tid] = 0;
@@ -1486,7 +1563,7 @@ __global__ __launch_bounds__(1024) void prefill_order(AttnArgs a) {
 template <int D>
 constexpr int merge_rows() { return 256 / (D / 4); }
 
-template <typename T, int D>
+template <typename T, int D, bool kDirect>
 __global__ __launch_bounds__(256) void prefill_merge(AttnArgs a) {
   constexpr int kLanes = D / 4;  // per row
   constexpr int kRows = merge_rows<D>();
@@ -1495,10 +1572,19 @@ __global__ __launch_bounds__(256) void prefill_merge(AttnArgs a) {
   const int i = (int)(blockIdx.x / (unsigned)(a.num_kv_heads * chunks));
   const int kvh = (int)(blockIdx.x / (unsigned)chunks % (unsigned)a.num_kv_heads);
   const int chunk = (int)(blockIdx.x % (unsigned)chunks);
-  if (i >= a.queue[kPrefillQueues + 2]) return;
-  const int e = a.split_first[i];
-  const int p = a.work_range[e].w;
-  const int4 en = a.work[e];
+  int e, p;
+  int4 en;
+  if constexpr (kDirect) {
+    int4 range;
+    en = direct_split_entry<true>(a, i, range, e);
+    if (en.x < 0) return;
+    p = range.w;
+  } else {
+    if (i >= a.queue[kPrefillQueues + 2]) return;
+    e = a.split_first[i];
+    p = a.work_range[e].w;
+    en = a.work[e];
+  }
   const int bq = a.block_q, G = a.groups;
   const int qb = en.x % a.num_qblocks;
   const int nq = en.z;
@@ -1583,7 +1669,7 @@ bool prefill_mfma_applies(const AttnArgs& a, int dtype) {
 
 // `rows`: the one-query rows' decode split to run in the same launch
 // (prefill_pp_rows), or null.
-static int launch_prefill_merge(const AttnArgs& a, int dtype, hipStream_t s);
+static int launch_prefill_merge(const AttnArgs& a, int dtype, hipStream_t s, bool direct);
 
 template <int W>
 static int launch_prefill_waves(AttnArgs a, int dtype, hipStream_t s, const AttnArgs* rows) {
@@ -1611,9 +1697,16 @@ static int launch_prefill_waves(AttnArgs a, int dtype, hipStream_t s, const Attn
   // A small pass whose every unit fits the grid at once needs no order: one
   // work-group per unit, each finding its own, one launch.
   const int64_t full = (device_cu_count() + kPrefillQueues - 1) / kPrefillQueues * kPrefillQueues;
-  const bool direct = !rows && !a.split_ok && a.batch <= kPrefillDirectBatch && units <= full;
+  // A split pass of head_dim 64 is direct too (its pieces are at most the
+  // grid's units): against the list's, 30.0 -> 26.6 us for 100 queries over
+  // 4,096 keys, 47.5 -> 41.8 for 512 over 4,096, 37.3 -> 30.1 for 64 over
+  // 15,000 (bf16, 32 / 8 heads). At head_dim 128 a large one loses what a
+  // small one gains (64 over 1,024: 33.3 -> 31.6; 1,000 over 6,000: 128.2 ->
+  // 129.2), so it keeps the list.
+  const bool direct =
+      !rows && a.batch <= kPrefillDirectBatch && units <= full && (!a.split_ok || a.head_dim == 64);
   if (direct) {
-    grid = units;  // a multiple of the queue count (every KV head has a unit of each block)
+    if (!a.split_ok) grid = units;  // a multiple of the queue count (every KV head has a unit of each block)
   } else {
     hipLaunchKernelGGL(prefill_order, dim3(1), dim3(1024), 0, s, a);
     if (int rc = check_launch("prefill_order")) return rc;
@@ -1641,7 +1734,7 @@ static int launch_prefill_waves(AttnArgs a, int dtype, hipStream_t s, const Attn
     }
 #undef LI_PP_ROWS
     if (int rc = check_launch("prefill_pp_rows")) return rc;
-    if (int rc = launch_prefill_merge(a, dtype, s)) return rc;
+    if (int rc = launch_prefill_merge(a, dtype, s, false)) return rc;
     return launch_combine_balanced(*rows, dtype, s);
   }
   if (a.kv_fp8) {
@@ -1655,7 +1748,8 @@ static int launch_prefill_waves(AttnArgs a, int dtype, hipStream_t s, const Attn
   } else {
 #define LI_PP(T, D)                                                                                 \
   do {                                                                                              \
-    if (a.split_ok) hipLaunchKernelGGL((prefill_pp<T, D, true, false>), g, block, 0, s, a);         \
+    if (a.split_ok && direct) hipLaunchKernelGGL((prefill_pp<T, 64, true, true>), g, block, 0, s, a); \
+    else if (a.split_ok) hipLaunchKernelGGL((prefill_pp<T, D, true, false>), g, block, 0, s, a);    \
     else if (direct) hipLaunchKernelGGL((prefill_pp<T, D, false, true>), g, block, 0, s, a);        \
     else hipLaunchKernelGGL((prefill_pp<T, D, false, false>), g, block, 0, s, a);                   \
   } while (0)
@@ -1669,23 +1763,29 @@ static int launch_prefill_waves(AttnArgs a, int dtype, hipStream_t s, const Attn
 #undef LI_PP
   }
   if (int rc = check_launch("prefill_mfma")) return rc;
-  return launch_prefill_merge(a, dtype, s);
+  return launch_prefill_merge(a, dtype, s, direct);
 }
 
 // After a pass that may be split: one work-group per (work-list entry that
 // can hold a piece, KV head); those of a split block's first piece fold it.
-static int launch_prefill_merge(const AttnArgs& a, int dtype, hipStream_t s) {
+static int launch_prefill_merge(const AttnArgs& a, int dtype, hipStream_t s, bool direct) {
   if (!a.split_ok) return LI_OK;
   const int chunks = kMinRows / (a.head_dim == 128 ? merge_rows<128>() : merge_rows<64>());
   const dim3 g((unsigned)(prefill_split_blocks_cap(a.split_target, a.num_kv_heads) * a.num_kv_heads * chunks)),
       block(256);
+#define LI_MERGE(T, D)                                                                       \
+  do {                                                                                       \
+    if (direct) hipLaunchKernelGGL((prefill_merge<T, 64, true>), g, block, 0, s, a);         \
+    else hipLaunchKernelGGL((prefill_merge<T, D, false>), g, block, 0, s, a);                \
+  } while (0)  // (direct: head_dim 64)
   if (dtype == LI_BF16) {
-    if (a.head_dim == 128) hipLaunchKernelGGL((prefill_merge<li_bf16, 128>), g, block, 0, s, a);
-    else hipLaunchKernelGGL((prefill_merge<li_bf16, 64>), g, block, 0, s, a);
+    if (a.head_dim == 128) LI_MERGE(li_bf16, 128);
+    else LI_MERGE(li_bf16, 64);
   } else {
-    if (a.head_dim == 128) hipLaunchKernelGGL((prefill_merge<li_f16, 128>), g, block, 0, s, a);
-    else hipLaunchKernelGGL((prefill_merge<li_f16, 64>), g, block, 0, s, a);
+    if (a.head_dim == 128) LI_MERGE(li_f16, 128);
+    else LI_MERGE(li_f16, 64);
   }
+#undef LI_MERGE
   return check_launch("prefill_merge");
 }
 
