@@ -32,7 +32,7 @@
 // a causal block's work is even) and merge their softmax states in LDS, as
 // the reference's cross-partition reduce does (paged_kernels.py:574-629).
 //
-// Measured (MI355X), three chukF32Waves of 281 .. 336 queries over 300 .. 1,100
+// Measured (MI355X), three chunks of 281 .. 336 queries over 300 .. 1,100
 // cached keys beside five one-query rows, 32 / 8 heads, head_dim 64 (7.1
 // GFLOP, 51 us at the rate of a large fp32 GEMM): 94 us, against 35.5 ms on
 // the general-shape kernel. What is left is a unit's start and end (its
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(
   // query counts, the last block of a sequence (most keys) first; a grid of
   // about twice what the GPU holds walks them. (A grid sized by the longest
   // chunk is mostly empty beside short ones, and an empty work-group costs
-  // its launch: 27 us for 2,990 of them beside three 300-query chukF32Waves.)
+  // its launch: 27 us for 2,990 of them beside three 300-query chunks.)
   const int kvh = (int)(blockIdx.x % (unsigned)a.num_kv_heads);
   // The first 64 sequences' query rows and blocks, kept for every unit.
   auto info_of = [&](int sq, int& first, int& count) -> int {  // returns the sequence's blocks

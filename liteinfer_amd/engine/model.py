@@ -12,8 +12,9 @@ reference's three `nn.Linear`s stacked, the same products), RoPE and the KV
 slot-write in one HIP launch (`payload.update_rotated`, the fused form of
 llama.py:155-160), `paged_attention` (llama.py:161), the output projection,
 RMSNorm and the SiLU-gated MLP (llama.py:101-112) with gate and up stacked.
-Projections are torch GEMMs (hipBLASLt); attention, RoPE and the slot-write are
-this library's kernels.
+On a ROCm device 16-bit projections of up to 256 rows run as this library's
+kernels where those are the faster ones (engine/ops.py), the others as torch
+GEMMs (hipBLASLt); attention, RoPE and the slot-write are this library's kernels.
 """
 
 from __future__ import annotations
