@@ -322,8 +322,11 @@ __global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(
       spread(s1, vs);
       issue_k_f32<D>(knext, kpool, vs, row_bytes, n, g);
       load_v_f32<D>(vnext, vpool, vs, row_bytes, n);
-      // The tile's K has landed once at most this step's loads (a slot, 4 kH
-      // of K, 4 kH of V) are in flight: they are all newer.
+      // Newer than the tile's K: its V (4 kH loads), this step's slot, K and
+      // V (1 + 8 kH). With 8 kH + 1 in flight its K has landed, and needs no
+      // more of this step's loads for that than K's (assembly, never dropped)
+      // and one other: a step whose look-ahead nobody reads may not use this
+      // count, since the compiler drops such loads.
       li_wait_vm<8 * kH + 1>();
       // (Left to itself the scheduler sikF32Waves the loads between the MFMAs.)
       __builtin_amdgcn_sched_barrier(0);
@@ -339,8 +342,14 @@ __global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(
       step(stage0, va, stage1, vn, sa, sb);
       step(stage1, vn, stage0, va, sb, sa);
     }
-    if (tile < clear) step(stage0, va, stage1, vn, sa, sb);
+    // The odd tile has nothing to look ahead to.
     li_wait_vm<0>();
+    __builtin_amdgcn_sched_barrier(0);
+    if (tile < clear) {
+      fold(std::false_type{}, stage0, va, sa, kb + 16 * tile);
+      __builtin_amdgcn_sched_barrier(0);
+      tile += kF32Waves;
+    }
   }
   for (; tile < ntiles; tile += kF32Waves) {
     u32x4_t v[4][kH];
