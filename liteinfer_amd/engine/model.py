@@ -106,7 +106,7 @@ class RandomLlama:
 
     def _rotary(self, positions: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         """cos / sin ``[B, T, D]`` in the model dtype, computed in fp32 (llama.py:70-78)."""
-        if self._fused_ops:
+        if self._fused_ops and not positions.is_floating_point():
             return self._fused_ops.rotary_tables(positions, self.inv_freq, self.dtype)
         freqs = positions[..., None].to(torch.float32) * self.inv_freq
         emb = torch.cat((freqs, freqs), dim=-1)

@@ -4,8 +4,10 @@
 
 Same results as the model's torch ops (liteinfer/models/llama.py:34-48,
 :101-116) up to the order of the fp32 sum of squares and the exponential's
-last bit; one launch each instead of a chain of torch kernels. Refuse what
-they do not serve (ValueError); the model keeps its torch ops for CPU tensors.
+last bit; one launch each instead of a chain of torch kernels. The kernels
+read raw pointers, so every operand is checked here first: the projections
+leave what they do not serve to `F.linear`, which serves or refuses it, the
+others raise ValueError. The model keeps its torch ops for CPU tensors.
 """
 
 from __future__ import annotations
@@ -29,6 +31,13 @@ def _rows(t: torch.Tensor, name: str) -> tuple[int, int]:
     return flat.shape[0], (flat.stride(0) if flat.shape[0] > 1 else t.shape[-1])
 
 
+def _same_device(what: str, *tensors: torch.Tensor) -> torch.device:
+    device = tensors[0].device
+    if device.type != "cuda" or any(t.device != device for t in tensors[1:]):
+        raise ValueError(f"{what} takes tensors on one ROCm device, got {[str(t.device) for t in tensors]}")
+    return device
+
+
 class Partials(NamedTuple):
     """A projection as fp32 sums over runs of its K, ``[splits, rows, n]``: what an op that follows adds and rounds."""
 
@@ -46,7 +55,7 @@ SKINNY_MAX_ROWS = 256
 @functools.lru_cache(maxsize=4096)
 def _splits(rows: int, n: int, k: int) -> int:
     """Runs of K one projection is cut into (0: torch's GEMM serves it)."""
-    if rows > SKINNY_MAX_ROWS or n % 8 or k % 128:
+    if rows > SKINNY_MAX_ROWS or n % 8 or k % 128 or not n or not k:
         return 0
     splits = ctypes.c_int()
     status = _native.load().li_skinny_gemm_plan(rows, n, k, ctypes.byref(splits))
@@ -57,7 +66,10 @@ def _splits(rows: int, n: int, k: int) -> int:
 
 
 def _skinny(x: torch.Tensor, w: torch.Tensor) -> tuple[torch.Tensor, int]:
-    """x as ``[rows, k]`` and the splits of ``x @ w.T`` (0: not this kernel's)."""
+    """x as ``[rows, k]`` and the splits of ``x @ w.T`` (0: not this kernel's, and x as it came)."""
+    if (not x.is_cuda or w.device != x.device or x.dim() < 1 or w.dim() != 2 or x.shape[-1] != w.shape[1]
+            or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))):
+        return x, 0
     flat = x.reshape(-1, x.shape[-1])
     if (x.dtype not in (torch.bfloat16, torch.float16) or w.dtype != x.dtype or not w.is_contiguous()
             or flat.stride(-1) != 1 or flat.stride(0) % 8 or flat.data_ptr() % 16 or w.data_ptr() % 16):
@@ -128,8 +140,13 @@ def add_rms_norm(h: torch.Tensor, weight: torch.Tensor, eps: float,
         raise ValueError("add_rms_norm takes bf16 / f16 rows and a weight of their width and dtype")
     if delta is not None and (delta.shape != h.shape or (not isinstance(delta, Partials) and delta.dtype != h.dtype)):
         raise ValueError("delta must match h")
+    _same_device("add_rms_norm", h, weight, *(() if delta is None else (delta.sums if isinstance(delta, Partials) else delta,)))
     rows, h_s = _rows(h, "h")
     if isinstance(delta, Partials):
+        if (delta.sums.dtype != torch.float32 or delta.sums.dim() != 3 or not delta.sums.is_contiguous()
+                or delta.sums.shape[1:] != (rows, h.shape[-1])):
+            raise ValueError(f"partial sums must be contiguous float32 [splits, {rows}, {h.shape[-1]}], "
+                             f"got {delta.sums.dtype} {list(delta.sums.shape)}")
         out = torch.empty(h.shape, dtype=h.dtype, device=h.device)
         status = _native.load().li_add_rms_norm_partials(
             h.data_ptr(), delta.sums.data_ptr(), delta.sums.shape[0], weight.contiguous().data_ptr(), out.data_ptr(),
@@ -151,6 +168,7 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     """``silu(gate) * up`` of the fused projection's halves ``gate_up = [gate | up]``."""
     if gate_up.dtype not in (torch.bfloat16, torch.float16) or gate_up.shape[-1] % 2:
         raise ValueError("silu_mul takes bf16 / f16 rows of an even width")
+    _same_device("silu_mul", gate_up)
     ffn = gate_up.shape[-1] // 2
     rows, gu_s = _rows(gate_up, "gate_up")
     out = torch.empty(*gate_up.shape[:-1], ffn, dtype=gate_up.dtype, device=gate_up.device)
@@ -162,6 +180,11 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
 
 def rotary_tables(positions: torch.Tensor, inv_freq: torch.Tensor, dtype: torch.dtype) -> tuple[torch.Tensor, torch.Tensor]:
     """cos / sin ``[..., D]`` of `positions` times `inv_freq` (``[D / 2]`` fp32, each twice), rounded to `dtype`."""
+    _same_device("rotary_tables", positions, inv_freq)
+    if positions.is_floating_point() or positions.is_complex():
+        raise ValueError(f"rotary_tables takes whole positions, got {positions.dtype}")
+    if inv_freq.dtype != torch.float32 or inv_freq.dim() != 1 or not inv_freq.is_contiguous():
+        raise ValueError(f"inv_freq must be contiguous float32 [D / 2], got {inv_freq.dtype} {list(inv_freq.shape)}")
     positions = positions.to(torch.int64).contiguous()
     half = inv_freq.shape[0]
     cos, sin = (torch.empty(*positions.shape, 2 * half, dtype=dtype, device=positions.device) for _ in range(2))
@@ -180,7 +203,16 @@ def stage_decode(inputs: tuple[torch.Tensor, ...], static: tuple[torch.Tensor, .
     """
     ids, positions, write_slots, slots, lens = inputs
     n, cols = slots.shape
-    device = static[0].device
+    device = _same_device("stage_decode", *static)
+    ids_out, positions_out, write_out, table_out, lens_out = static
+    for t in (ids_out, positions_out, write_out, lens_out):
+        if t.numel() < width or not t.is_contiguous() or t.dtype != (torch.int32 if t is lens_out else torch.int64):
+            raise ValueError(f"the static columns must be contiguous int64 (lengths int32) of at least {width} rows, "
+                             f"got {t.dtype} {list(t.shape)}")
+    if (table_out.dtype != torch.int64 or table_out.dim() != 2 or table_out.stride(1) != 1 or n > width
+            or width > table_out.shape[0] or max(cols, 1) > table_out.shape[1] or table_out.stride(0) < table_out.shape[1]):
+        raise ValueError(f"a step of {n} x {cols} slots, padded to {width} rows, does not fit a "
+                         f"{list(table_out.shape)} {table_out.dtype} slot table")
 
     def column(t: torch.Tensor, shape: tuple[int, ...], dtype: torch.dtype) -> torch.Tensor:
         return torch.broadcast_to(t, shape).to(device=device, dtype=dtype).contiguous()
@@ -192,6 +224,6 @@ def stage_decode(inputs: tuple[torch.Tensor, ...], static: tuple[torch.Tensor, .
         slots = slots.contiguous()
     status = _native.load().li_stage_decode(
         ids.data_ptr(), positions.data_ptr(), write_slots.data_ptr(), slots.data_ptr(), slots.stride(0), lens.data_ptr(),
-        static[0].data_ptr(), static[1].data_ptr(), static[2].data_ptr(), static[3].data_ptr(), static[3].stride(0),
-        static[4].data_ptr(), n, cols, width, pad_slot, _native.stream_handle(device))
+        ids_out.data_ptr(), positions_out.data_ptr(), write_out.data_ptr(), table_out.data_ptr(), table_out.stride(0),
+        lens_out.data_ptr(), n, cols, width, pad_slot, _native.stream_handle(device))
     _native.check(status, "stage_decode")
