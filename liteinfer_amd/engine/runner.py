@@ -121,10 +121,10 @@ class DecodeGraphs:
 
     def run(self, input_ids, positions, write_slots, slots, context_lens) -> torch.Tensor:
         n, cols = slots.shape
-        width = self._width_for(n)
         if n > self.slot_table.shape[0] or cols > self.slot_table.shape[1]:
             raise ValueError(f"a step of {n} x {cols} slots does not fit the captured "
                              f"{tuple(self.slot_table.shape)} table")
+        width = self._width_for(n)
         stage_decode((input_ids, positions, write_slots, slots, context_lens),
                      (self.input_ids, self.positions, self.write_slots, self.slot_table, self.context_lens),
                      width, self.pad_slot)

@@ -15,6 +15,7 @@ import torch.nn.functional as F
 
 from liteinfer_amd.engine import ops
 from liteinfer_amd.engine.model import RandomLlama
+from liteinfer_amd.engine.runner import DecodeGraphs
 
 
 class _OnGpu(torch.Tensor):
@@ -147,3 +148,10 @@ def test_a_step_that_does_not_fit_its_buffers_is_refused(n, cols, width, change)
     inputs = tuple(torch.zeros(*s, dtype=torch.int64) for s in ((n, 1), (n, 1), (1, n), (n, cols), (n,)))
     with pytest.raises(ValueError):
         ops.stage_decode(inputs, tuple(static), width, 0)
+
+
+@pytest.mark.parametrize("n,cols", [(5, 3), (2, 17)])
+def test_a_step_larger_than_the_captured_buffers_is_refused(n, cols):
+    graphs = DecodeGraphs(SimpleNamespace(device=torch.device("cpu")), None, max_num_seqs=4, max_model_len=16, pad_slot=0)
+    with pytest.raises(ValueError, match="does not fit the captured"):
+        graphs.run(None, None, None, torch.zeros(n, cols, dtype=torch.int64), None)
