@@ -383,13 +383,15 @@ __global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(
     float mx = -INFINITY;
 #pragma unroll
     for (int v = 0; v < kF32Waves; ++v) mx = fmaxf(mx, s_m[v][rr]);
+    // A wave that met none of the row's keys holds m = -inf and zero sums. So
+    // does one whose scores were all NaN, but for its sums: every wave's are
+    // added, whatever its m, so that a NaN reaches the row.
+    const float base = mx == -INFINITY ? 0.f : mx;
     floatx4_t num = {0.f, 0.f, 0.f, 0.f};
     float den = 0.f;
 #pragma unroll
     for (int v = 0; v < kF32Waves; ++v) {
-      // A wave that met none of the row's keys holds m = -inf and zero sums.
-      if (s_m[v][rr] == -INFINITY) continue;
-      const float wgt = __builtin_amdgcn_exp2f(s_m[v][rr] - mx);
+      const float wgt = __builtin_amdgcn_exp2f(s_m[v][rr] - base);
       den = fmaf(wgt, s_l[v][rr], den);
       const floatx4_t x = *reinterpret_cast<const floatx4_t*>(&lds.acc[v][rr][4 * c]);
 #pragma unroll

@@ -75,3 +75,42 @@ def test_an_empty_context_is_nan():
     lens = torch.tensor([0, 9], dtype=torch.int32, device="cuda")
     out = paged_decode(b.query, b.key_pool, b.value_pool, b.slot_table, lens, b.scaling, b.groups)
     assert torch.isnan(out[0]).all() and torch.isfinite(out[1]).all()
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("ctx", [1, 16, 17, 33, 49, 65, 1000])
+@pytest.mark.parametrize("num_splits", [None, 3])
+def test_a_nan_in_the_newest_key_reaches_the_result(ctx, num_splits, head_dim):
+    """At 17, 33 and 49 keys one wave's only key is the newest, so every score that it sees is a NaN."""
+    b = PagedBatch([ctx, 50], num_heads=8, num_kv_heads=2, head_dim=head_dim, num_slots=2048)
+    b.slot_table = torch.arange(2 * max(ctx, 50), device="cuda").reshape(2, -1)
+    b.key_pool[ctx - 1, 0] = float("nan")  # of the first KV head
+    out = paged_decode(b.query, b.key_pool, b.value_pool, b.slot_table, b.context_lens_t, b.scaling, b.groups,
+                       num_splits=num_splits)
+    assert torch.isnan(out[0, :4]).all() and torch.isfinite(out[0, 4:]).all() and torch.isfinite(out[1]).all()
+
+
+def test_a_packed_row_sees_a_nan_key_of_its_own():
+    """The last query alone sees the last key, which is a tile and one wave's whole share."""
+    b = PagedBatch([17, 33], [2, 3], num_heads=2, num_kv_heads=2, head_dim=64)
+    b.slot_table = torch.arange(66, device="cuda").reshape(2, 33)
+    want = _prefill(b)
+    b.key_pool[[16, 65]] = float("nan")
+    got = _prefill(b)
+    assert torch.isnan(got[[1, 4]]).all()
+    np.testing.assert_allclose(to_numpy(got[[0, 2, 3]]), to_numpy(want[[0, 2, 3]]), rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("ctx", [17, 40])
+def test_infinite_scores(ctx):
+    """A newest key of an infinite score: minus infinity weighs nothing, plus infinity is a NaN."""
+    b = PagedBatch([ctx], num_heads=8, num_kv_heads=2, head_dim=64)
+    b.slot_table = torch.arange(ctx, device="cuda").reshape(1, ctx)
+    b.key_pool[ctx - 1, :, 0] = float("inf")
+    args = (b.scaling, b.groups)
+    got = paged_decode(b.query, b.key_pool, b.value_pool, b.slot_table, b.context_lens_t, *args)
+    without = paged_decode(b.query, b.key_pool, b.value_pool, b.slot_table, b.context_lens_t - 1, *args)
+    up = b.query[0, :, 0] > 0
+    assert up.any() and not up.all()
+    assert torch.isnan(got[0, up]).all()
+    np.testing.assert_allclose(to_numpy(got[0, ~up]), to_numpy(without[0, ~up]), rtol=1e-5, atol=1e-5)
