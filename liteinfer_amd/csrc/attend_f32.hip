@@ -428,17 +428,20 @@ bool rows_aligned(const void* p, int64_t s0, int64_t s1) {
 }  // namespace
 
 bool attend_f32_applies(const AttnArgs& a, int dtype) {
+  // A decode step has a work-group for every unit, and a launch fewer than
+  // 2^32 threads: past that the general kernel's smaller work-groups still fit.
+  // (A packed pass's grid is capped.)
+  const int64_t units = (int64_t)a.batch * a.num_parts * a.num_kv_heads * cdiv(a.groups, kF32Rows);
+  if (!a.qsl && units >= (1LL << 32) / (64 * kF32Waves)) return false;
   return dtype == LI_F32 && !a.kv_fp8 && (a.head_dim == 64 || a.head_dim == 128) && rows_aligned(a.q, a.q_s0, a.q_s1) &&
          rows_aligned(a.out, a.o_s0, a.o_s1) && rows_aligned(a.kp, a.p_s0, a.p_s1) &&
          rows_aligned(a.vp, a.p_s0, a.p_s1) && a.p_s0 >= 0 && a.p_s0 < (1LL << 30);
 }
 
 int launch_attend_f32(AttnArgs a, hipStream_t s) {
-  a.num_qblocks = (int)cdiv64((int64_t)std::max(a.max_query_len, 1) * a.groups, kF32Rows);
+  a.num_qblocks = (int)std::min<int64_t>(cdiv64((int64_t)std::max(a.max_query_len, 1) * a.groups, kF32Rows), 0x7fffffff);
   const int64_t most = (int64_t)a.batch * a.num_qblocks * a.num_parts;
   if (most == 0) return LI_OK;
-  if (most * a.num_kv_heads > 0x7fffffffLL)
-    return fail(LI_EUNSUPPORTED, "attention grid of %lld blocks is too large", (long long)(most * a.num_kv_heads));
   int64_t per_head = most;
   if (a.qsl) {
     // About twice what the CUs hold at once (two or three each): the first

@@ -114,3 +114,21 @@ def test_infinite_scores(ctx):
     assert up.any() and not up.all()
     assert torch.isnan(got[0, up]).all()
     np.testing.assert_allclose(to_numpy(got[0, ~up]), to_numpy(without[0, ~up]), rtol=1e-5, atol=1e-5)
+
+
+def test_the_longest_chunk_may_be_overstated():
+    """`max_query_len` bounds the chunks; the grid does not grow with what it overstates."""
+    b = PagedBatch([20, 9], [3, 9], num_heads=32, num_kv_heads=2, head_dim=64)
+    got = paged_prefill(b.query, b.key_pool, b.value_pool, b.slot_table, b.context_lens_t, b.query_start_loc,
+                        2 ** 31 - 1, b.scaling, b.groups)
+    assert torch.equal(got, _prefill(b))
+
+
+def test_a_decode_step_of_more_units_than_a_launch_holds():
+    """2^24 units of 256 threads are past a launch's 2^32: the general kernel serves them."""
+    batch, heads = 2 ** 24 // 32, 32
+    b = PagedBatch([1], num_heads=heads, num_kv_heads=heads, head_dim=64)
+    table = torch.arange(batch, device="cuda").remainder(512).view(batch, 1)
+    lens = torch.ones(batch, dtype=torch.int32, device="cuda")
+    out = paged_decode(b.query.expand(batch, heads, 64), b.key_pool, b.value_pool, table, lens, b.scaling, 1)
+    assert torch.equal(out.view(-1, 512, heads, 64), b.value_pool.expand(batch // 512, 512, heads, 64))
