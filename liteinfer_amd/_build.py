@@ -2,9 +2,11 @@
 
 Every ``csrc/*.hip`` file is compiled for gfx950 by ``hipcc`` and linked into
 one shared library with a plain C ABI (``include/liteinfer_amd.h``). The
-library is loaded with ctypes, so nothing here depends on torch's extension
-machinery; it links the HIP runtime by soname, which resolves to the copy the
-process already has loaded when torch was imported first.
+library is loaded with ctypes and depends on no torch; it links the HIP runtime
+by soname, which resolves to the copy the process already has loaded when
+torch was imported first. Beside it the host compiler builds
+``csrc/fast_calls.cpp``, a Python extension against this interpreter and its
+torch, whose file name carries a digest of both.
 
 Run as ``python -m liteinfer_amd._build``.
 """
@@ -24,7 +26,6 @@ PACKAGE_DIR = Path(__file__).resolve().parent
 CSRC_DIR = PACKAGE_DIR / "csrc"
 LIB_DIR = PACKAGE_DIR / "_lib"
 LIB_PATH = LIB_DIR / "libliteinfer_amd.so"
-FAST_CALLS_PATH = LIB_DIR / "_fast_calls.so"
 INCLUDE_DIR = PACKAGE_DIR.parent / "include"
 
 OFFLOAD_ARCH = "gfx950"
@@ -96,6 +97,27 @@ def _compile(src: Path, obj: Path, build_id: str) -> None:
         print(err, file=sys.stderr)
 
 
+# Host flags and libraries of csrc/fast_calls.cpp.
+FAST_CALLS_FLAGS = ["-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-w"]
+FAST_CALLS_LIBS = ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
+
+
+def fast_calls_path() -> Path:
+    """Where the extension for this interpreter and this torch lies.
+
+    Its code reads torch's and Python's objects at offsets fixed when it was
+    compiled, so the name carries a digest of what these depend on: an
+    extension built for others is not found.
+    """
+    import sysconfig
+
+    import torch
+
+    abi = (torch.__version__, torch.version.git_version, torch._C._GLIBCXX_USE_CXX11_ABI, sys.implementation.cache_tag,
+           sysconfig.get_config_var("SOABI"), FAST_CALLS_FLAGS, FAST_CALLS_LIBS)
+    return LIB_DIR / f"_fast_calls.{hashlib.sha256(repr(abi).encode()).hexdigest()[:16]}.so"
+
+
 def _compile_fast_calls(build_id: str) -> None:
     """csrc/fast_calls.cpp, the eager calls' host side: a Python extension against this interpreter's torch."""
     import sysconfig
@@ -103,17 +125,19 @@ def _compile_fast_calls(build_id: str) -> None:
     import torch
     from torch.utils import cpp_extension
 
+    path = fast_calls_path()
+    for stale in LIB_DIR.glob("_fast_calls*"):
+        stale.unlink()
     torch_lib = Path(torch.__file__).resolve().parent / "lib"
-    out_tmp = LIB_DIR / (FAST_CALLS_PATH.name + ".tmp")
-    cmd = [shutil.which("g++") or "c++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-w",
+    out_tmp = LIB_DIR / (path.name + ".tmp")
+    cmd = [shutil.which("g++") or "c++", *FAST_CALLS_FLAGS,
            f'-DLI_BUILD_ID="{build_id}"', f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            *(f"-I{p}" for p in (*cpp_extension.include_paths(), sysconfig.get_paths()["include"])),
-           str(CSRC_DIR / "fast_calls.cpp"), "-o", str(out_tmp),
-           f"-L{torch_lib}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
+           str(CSRC_DIR / "fast_calls.cpp"), "-o", str(out_tmp), f"-L{torch_lib}", *FAST_CALLS_LIBS]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"{cmd[0]} failed on fast_calls.cpp:\n{proc.stderr}")
-    os.replace(out_tmp, FAST_CALLS_PATH)
+    os.replace(out_tmp, path)
 
 
 def build(verbose: bool = False) -> Path:

@@ -204,7 +204,7 @@ def fast_calls():
     lib = load()
     with _lock:
         if _fast is None:
-            path = _build.FAST_CALLS_PATH
+            path = _build.fast_calls_path()
             if not path.exists():
                 raise NativeLibraryMissing(f"{path} is missing; run `python -m liteinfer_amd._build`")
             loader = importlib.machinery.ExtensionFileLoader("_fast_calls", str(path))

@@ -52,3 +52,17 @@ def test_a_module_of_other_sources_is_refused(monkeypatch):
     monkeypatch.setattr(_native, "load", lambda: object())
     with pytest.raises(RuntimeError, match="built from other sources"):
         _native.fast_calls()
+
+
+@pytest.mark.parametrize("owner,name,value", [
+    (torch, "__version__", "9.9.9"), (torch.version, "git_version", "f" * 40),
+    (torch._C, "_GLIBCXX_USE_CXX11_ABI", not torch._C._GLIBCXX_USE_CXX11_ABI),
+    (_native._build.sys.implementation, "cache_tag", "cpython-99"), (_native._build, "FAST_CALLS_FLAGS", ["-O3"]),
+])
+def test_a_module_for_another_torch_or_interpreter_is_not_found(monkeypatch, owner, name, value):
+    built = _native._build.fast_calls_path()
+    assert built.exists()
+    monkeypatch.setattr(owner, name, value)
+    assert not _native._build.fast_calls_path().exists()
+    monkeypatch.undo()
+    assert _native._build.fast_calls_path() == built
