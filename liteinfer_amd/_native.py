@@ -12,6 +12,7 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import threading
+import warnings
 from pathlib import Path
 
 import torch
@@ -193,10 +194,30 @@ def load() -> ctypes.CDLL:
 _fast = None
 
 
+class _PythonCalls:
+    """Stands for the extension where it cannot be loaded: every call is left to the Python code."""
+
+    @staticmethod
+    def decode(*_args):
+        return None
+
+    prefill = rope = decode
+
+
+def _load_fast_calls(path: Path):
+    loader = importlib.machinery.ExtensionFileLoader("_fast_calls", str(path))
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_fast_calls", loader))
+    loader.exec_module(module)
+    return module
+
+
 def fast_calls():
     """The eager calls' host side in C++ (``csrc/fast_calls.cpp``), bound to the loaded library.
 
     Its functions return None for every call they leave to the Python code.
+    Where it is not built for this torch and interpreter, or does not load, a
+    warning says so once and all calls are left to the Python code, which
+    serves them the same (some 15 us more on the host for a decode layer).
     """
     global _fast
     if _fast is not None:
@@ -205,11 +226,13 @@ def fast_calls():
     with _lock:
         if _fast is None:
             path = _build.fast_calls_path()
-            if not path.exists():
-                raise NativeLibraryMissing(f"{path} is missing; run `python -m liteinfer_amd._build`")
-            loader = importlib.machinery.ExtensionFileLoader("_fast_calls", str(path))
-            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_fast_calls", loader))
-            loader.exec_module(module)
+            try:
+                module = _load_fast_calls(path)
+            except ImportError as e:
+                warnings.warn(f"the eager calls' C++ host side cannot be loaded ({e}); they run through Python. "
+                              "Build it with `python -m liteinfer_amd._build`", RuntimeWarning, stacklevel=3)
+                _fast = _PythonCalls
+                return _fast
             expected = _build.source_hash()
             if module.build_id != expected:
                 raise RuntimeError(f"{path} was built from other sources (build id {module.build_id}, the sources here "

@@ -6,6 +6,8 @@ and the public calls must raise what they raised before.
 
 from __future__ import annotations
 
+import warnings
+
 import pytest
 import torch
 
@@ -66,3 +68,34 @@ def test_a_module_for_another_torch_or_interpreter_is_not_found(monkeypatch, own
     assert not _native._build.fast_calls_path().exists()
     monkeypatch.undo()
     assert _native._build.fast_calls_path() == built
+
+
+def _cannot_load(path):
+    raise ImportError("undefined symbol")
+
+
+@pytest.mark.parametrize("break_it", [
+    lambda m, tmp: m.setattr(_native._build, "LIB_DIR", tmp),  # not there
+    lambda m, tmp: m.setattr(_native, "_load_fast_calls", _cannot_load),
+])
+def test_without_the_module_the_python_code_serves_every_call(monkeypatch, tmp_path, break_it):
+    monkeypatch.setattr(_native, "_fast", None)
+    break_it(monkeypatch, tmp_path)
+    with pytest.warns(RuntimeWarning, match="run through Python"):
+        f = _native.fast_calls()
+    assert f.decode(*_operands(), 0.125, 4) is None and f.prefill() is None and f.rope(1) is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _native.fast_calls() is f  # (said once)
+
+
+def test_a_failed_extension_build_does_not_end_the_build(monkeypatch, tmp_path, capsys):
+    build = _native._build
+    monkeypatch.setattr(build, "LIB_DIR", tmp_path)
+    monkeypatch.setattr(build, "LIB_PATH", tmp_path / "lib.so")
+    monkeypatch.setattr(build, "FAST_CALLS_FLAGS", ["--no-such-flag"])
+    monkeypatch.setattr(build, "sources", lambda: [build.CSRC_DIR / "kv_scatter.hip"])
+    (tmp_path / "_fast_calls.0.so").touch()
+    assert build.build().exists()
+    assert "will run through Python" in capsys.readouterr().err
+    assert not list(tmp_path.glob("_fast_calls*"))
