@@ -422,7 +422,7 @@ int li_silu_mul(const void* gate_up, void* out, int64_t rows, int ffn,
  *
  * li_skinny_gemm_plan reports the runs of k the call should be cut into to
  * fill the GPU (*splits), or LI_EUNSUPPORTED where a general GEMM is faster
- * (most shapes past 64 rows). With splits == 1 `out` receives
+ * (most shapes past 64 rows, some from 33 on). With splits == 1 `out` receives
  * the rounded rows; otherwise `partials`, [splits, m, n] fp32, the sums of
  * each run, for one of the *_partials calls (which add and round them as
  * their delta / gate_up) or li_skinny_reduce (which rounds them to rows).

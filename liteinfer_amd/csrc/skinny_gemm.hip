@@ -66,8 +66,10 @@ struct Cut {
   int tile, splits;
 };
 
-// Up to 64 rows every projection measured faster here than through hipBLASLt
-// (1.0 .. 3.0 times, 10 shapes of the 8B and 1B architectures). K is cut into
+// Up to 64 rows the projections of the 8B and 1B architectures measured faster
+// here than through hipBLASLt (1.0 .. 3.0 times; what does not: uneven_rounds,
+// and the sums of 33 .. 64 rows that nothing adds, `linear` in engine/ops.py).
+// K is cut into
 // as many runs as fill the GPU once, of at least two stages (of one, the sums
 // cost the norm more than the run saves: a step of 4 layers of the 1B
 // architecture at 24 rows 322 -> 312 us); not at all where
@@ -78,8 +80,9 @@ struct Cut {
 // Past 64 rows a work-group reads x as often as its weights, and the runs'
 // sums cost more than they did; what stays faster (us, this against
 // hipBLASLt's, the norm that adds the sums included):
-//   whole tiles at up to 128 rows: 28672 x 4096 with its gate 53 / 58 at 128
-//     rows (74 / 61 at 160), 32064 x 2048 30 / 34;
+//   whole tiles at up to 128 rows, where uneven_rounds allows: 28672 x 4096
+//     with its gate 53 / 58 at 128 rows (74 / 61 at 160), 32064 x 2048 30 /
+//     34, 128256 x 4096 217 / 233;
 //   runs of K no shorter than 768 of a weight no wider than twice its K:
 //     4096 x 14336 40 / 79 at 128 rows and 49 / 66 at 256, 6144 x 4096 24 / 25
 //     and 30 / 40 (4096 x 4096, runs of 512: 24 / 29 and 28 / 27; 3072 x 2048,
@@ -104,6 +107,29 @@ Cut cut_of(int m, int n, int k) {
     if (m <= 192 && k / runs(64, 1) >= kMinRun) return {64, runs(64, 1)};
   }
   return {0, 0};
+}
+
+// Past 32 rows a wide weight's 128-row tiles take a CU each, round by round,
+// and a last round that is nearly empty costs a whole one: hipBLASLt, whose
+// tiles follow the shape, is then the faster one, so the plan leaves those
+// to it. The lines, us here / hipBLASLt's (rounds of 256 tiles):
+//   65 .. 128 rows, K under 4096, up to two rounds: 33024 x 1024 (1.01) 31 /
+//     21, 40960 x 2048 (1.25) 50 / 44, 49152 x 3584 (1.5) 87 / 77, 61440 x
+//     2048 (1.9) 58 / 54; from two on 65536 x 2048 61 / 72, 128256 x 2048 123
+//     / 123;
+//   65 .. 128 rows, longer K, up to one and a half: 33024 x 4096 87 / 69,
+//     40960 x 4096 89 / 80; from there 49152 x 4096 92 / 101, 128256 x 4096
+//     217 / 233;
+//   33 .. 64 rows, up to one and a half: 40960 x 1024 23 / 21, 33024 x 3584 63
+//     / 56 (and 36864 x 4096 69 / 73); from there 57344 x 3584 74 / 77.
+// What is left on the wrong side: 65536 x 3072 at 128 rows 89 / 84, 98304 x
+// 1024 56 / 49. At 32 rows and fewer (64-row tiles, two a CU) every width was
+// faster here. Under K of 512 both are mostly a launch, and whichever is
+// ahead changes with the row count.
+bool uneven_rounds(int m, int n, int k) {
+  const int cus = li::device_cu_count(), t = (n + 127) / 128;
+  if (m <= kFewRows || k < 512 || t <= cus) return false;
+  return t < (m > kSkinnyRows && k < 4096 ? 2 * cus : cus * 3 / 2);
 }
 
 // Stores lane (m, g)'s four sums of a group of 16 outputs: 16 group + 4g ..
@@ -418,16 +444,22 @@ void launch_rows(const GemmArgs& a, hipStream_t s) {
 
 }  // namespace
 
-extern "C" int li_skinny_gemm_plan(int m, int n, int k, int* splits) {
-  li::clear_error();
+static int check_extents(int m, int n, int k) {
   if (m < 0 || n <= 0 || k <= 0) return li::fail(LI_EINVAL, "li_skinny_gemm_plan: bad extents (%d, %d, %d)", m, n, k);
   if (m > LI_SKINNY_MAX_ROWS || n % 8 || k % kStageK)
     return li::fail(LI_EUNSUPPORTED, "li_skinny_gemm: up to %d rows, n a multiple of 8, k of %d; got %d, %d, %d",
                     LI_SKINNY_MAX_ROWS, kStageK, m, n, k);
-  const Cut cut = cut_of(m, n, k);
-  if (cut.splits == 0)
+  if (cut_of(m, n, k).splits == 0)
     return li::fail(LI_EUNSUPPORTED, "li_skinny_gemm: %d rows of %d x %d are a general GEMM's", m, n, k);
-  if (splits) *splits = cut.splits;
+  return LI_OK;
+}
+
+extern "C" int li_skinny_gemm_plan(int m, int n, int k, int* splits) {
+  li::clear_error();
+  if (int rc = check_extents(m, n, k)) return rc;
+  if (uneven_rounds(m, n, k))
+    return li::fail(LI_EUNSUPPORTED, "li_skinny_gemm: %d rows of %d x %d run faster as a general GEMM", m, n, k);
+  if (splits) *splits = cut_of(m, n, k).splits;
   return LI_OK;
 }
 
@@ -436,7 +468,7 @@ extern "C" int li_skinny_gemm(const void* x, int64_t x_stride, const void* w, in
                               int dtype, void* stream) {
   li::clear_error();
   if (dtype != LI_BF16 && dtype != LI_F16) return li::fail(LI_EUNSUPPORTED, "li_skinny_gemm: bf16 or f16 only");
-  if (int rc = li_skinny_gemm_plan(m, n, k, nullptr)) return rc;
+  if (int rc = check_extents(m, n, k)) return rc;
   if (splits < 1 || splits > k / kStageK) return li::fail(LI_EINVAL, "li_skinny_gemm: %d splits of %d", splits, k);
   if (gate_up && n % 16) return li::fail(LI_EUNSUPPORTED, "li_skinny_gemm: gate / up halves must be multiples of 8");
   if (m == 0) return LI_OK;

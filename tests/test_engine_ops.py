@@ -155,3 +155,16 @@ def test_a_step_larger_than_the_captured_buffers_is_refused(n, cols):
     graphs = DecodeGraphs(SimpleNamespace(device=torch.device("cpu")), None, max_num_seqs=4, max_model_len=16, pad_slot=0)
     with pytest.raises(ValueError, match="does not fit the captured"):
         graphs.run(None, None, None, torch.zeros(n, cols, dtype=torch.int64), None)
+
+
+@pytest.mark.parametrize("rows,n,k,served", [
+    (128, 32768, 2048, True), (65, 24576, 1024, True),  # one round of 128-row tiles
+    (65, 32776, 2048, False), (128, 40960, 1024, False), (128, 65408, 3584, False), (65, 65536, 3584, True),
+    (96, 40960, 4096, False), (96, 49152, 4096, True), (128, 128256, 4096, True), (128, 128256, 2048, True),
+    (33, 40960, 1024, False), (64, 49024, 3584, False), (64, 49152, 1024, True), (32, 40960, 1024, True),
+    (128, 33000, 256, True), (128, 33024, 512, False),
+])
+def test_wide_weights_of_uneven_rounds_are_torchs(monkeypatch, rows, n, k, served):
+    """256 CUs take 128-row tiles round by round; a nearly empty last round is left to torch's GEMM."""
+    monkeypatch.undo()  # the rule itself
+    assert (ops._splits(rows, n, k) > 0) == served
