@@ -33,8 +33,9 @@ def _rows(t: torch.Tensor, name: str) -> tuple[int, int]:
 
 def _same_device(what: str, *tensors: torch.Tensor) -> torch.device:
     device = tensors[0].device
-    if device.type != "cuda" or any(t.device != device for t in tensors[1:]):
-        raise ValueError(f"{what} takes tensors on one ROCm device, got {[str(t.device) for t in tensors]}")
+    for t in tensors:
+        if not t.is_cuda or t.device != device:
+            raise ValueError(f"{what} takes tensors on one ROCm device, got {[str(t.device) for t in tensors]}")
     return device
 
 
@@ -215,6 +216,8 @@ def stage_decode(inputs: tuple[torch.Tensor, ...], static: tuple[torch.Tensor, .
                          f"{list(table_out.shape)} {table_out.dtype} slot table")
 
     def column(t: torch.Tensor, shape: tuple[int, ...], dtype: torch.dtype) -> torch.Tensor:
+        if t.shape == shape and t.dtype == dtype and t.device == device and t.is_contiguous():
+            return t  # (as the engine brings it: 0.6 us on the host, the conversions that change nothing 3)
         return torch.broadcast_to(t, shape).to(device=device, dtype=dtype).contiguous()
 
     ids, positions = column(ids, (n, 1), torch.int64), column(positions, (n, 1), torch.int64)
