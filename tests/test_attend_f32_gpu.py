@@ -1,9 +1,9 @@
 """fp32 attention on the fp32 matrix cores (head_dim 64 and 128) against the fp64 oracle.
 
-Sizes sit at the kernel's edges: 16-key tiles, 16-row groups and blocks of
-32 rows (with groupings that fill them oddly), a single key, more keys than
-four waves' tiles, pinned splits, and rows whose block reaches past keys they
-do not see. Bound: fp32's 1e-5 (the sums run over at most a few thousand
+Sizes sit at the kernel's edges: 16-key tiles, blocks of 16 rows (with
+groupings that fill them oddly), a single key, more keys than four waves'
+tiles, pinned splits, rows whose block reaches past keys they do not see,
+more blocks than work-groups, and more sequences than one scan covers. Bound: fp32's 1e-5 (the sums run over at most a few thousand
 products of N(0, 1) values, ~1e-6 off).
 """
 
@@ -132,3 +132,23 @@ def test_a_decode_step_of_more_units_than_a_launch_holds():
     lens = torch.ones(batch, dtype=torch.int32, device="cuda")
     out = paged_decode(b.query.expand(batch, heads, 64), b.key_pool, b.value_pool, table, lens, b.scaling, 1)
     assert torch.equal(out.view(-1, 512, heads, 64), b.value_pool.expand(batch // 512, 512, heads, 64))
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+def test_work_groups_take_several_units(head_dim):
+    """Blocks past the capped grid: 6 work-groups a CU over the KV heads walk them."""
+    q = [1, 400, 150, 97, 700]
+    b = PagedBatch([300, 410, 150, 160, 731], q, num_heads=32, num_kv_heads=8, head_dim=head_dim)
+    per_head = sum(-(-n * b.groups // 16) for n in q)
+    assert per_head > -(-torch.cuda.get_device_properties(0).multi_processor_count * 6 // 8)
+    _close(_prefill(b), b.oracle())
+
+
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("batch", [64, 65, 130])
+def test_packed_past_one_scan_of_the_sequences(batch, head_dim):
+    """64 sequences' counts a scan, some of them bringing no query, the last one the longest chunk."""
+    q = [(3, 0, 1, 17, 0)[i % 5] for i in range(batch - 1)] + [40]
+    ctx = [n + 7 * i % 60 + (n == 0) for i, n in enumerate(q)]
+    b = PagedBatch(ctx, q, num_heads=8, num_kv_heads=2, head_dim=head_dim)
+    _close(_prefill(b), b.oracle())

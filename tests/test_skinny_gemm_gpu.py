@@ -2,7 +2,8 @@
 
 Sizes at the kernel's edges: one row, the row blocks of 16 / 32 / 64 / 128 / 256
 and one past them, weight rows that fill no 128-row tile, one 128-k stage, and K cut
-into many runs. Bound: the product of N(0, 1) x and 0.02 N(0, 1) w in fp32,
+into many runs. `test_gate_up` also holds sizes that torch's GEMM serves;
+`test_gate_up_through_every_kernel` names the kernels' own. Bound: the product of N(0, 1) x and 0.02 N(0, 1) w in fp32,
 rounded once: half an ulp (at most 2^-8 relative in bf16, 2^-11 in fp16) plus fp32
 summation error, well under 1e-4 here.
 """
@@ -84,3 +85,24 @@ def test_rows_it_does_not_serve_run_as_torch_products():
     assert ops._skinny(x, w)[1] == 0
     odd = torch.zeros(4, 264, device="cuda", dtype=torch.bfloat16)[:, 4:260]
     assert ops._skinny(odd, torch.zeros(128, 256, device="cuda", dtype=torch.bfloat16))[1] == 0
+
+
+@pytest.mark.parametrize("rows,ffn,k,splits", [
+    (1, 1032, 512, 2), (24, 2048, 2048, 8), (64, 1032, 512, 2),  # skinny_gemm's gated sums
+    (65, 2048, 4096, 4), (128, 2040, 4096, 4), (129, 2048, 4096, 4), (192, 2040, 4096, 4),  # 64-row tiles of batch_gemm
+    (65, 2048, 14336, 8), (128, 2040, 14336, 8), (129, 2040, 14336, 8), (256, 2048, 14336, 8),  # 128-row tiles
+    (65, 14336, 512, 1), (128, 12296, 512, 1),  # and whole ones, gated in the kernel
+])
+def test_gate_up_through_every_kernel(rows, ffn, k, splits):
+    """Against float64, over the routes that the rule of the cut takes."""
+    x, w, want = _inputs(rows, 2 * ffn, k, torch.bfloat16)
+    assert ops._skinny(x, w)[1] == splits
+    got = ops.gate_up_silu(x, w).double()
+    gate, up = want.chunk(2, -1)
+    out = F.silu(gate) * up
+    # Half a spacing each for up, the gate's value and the product; the gate's
+    # own moves silu by up to 1 + |gate| times as much. The fp32 sums: k terms
+    # of ~0.02, under 1e-4.
+    tol = (4 + gate.abs()) * 0.5 * ULP[torch.bfloat16] * out.abs() + 1e-4 * (1 + gate.abs() + up.abs())
+    err = (got - out).abs()
+    assert (err <= tol).all(), (err / tol).max()
