@@ -37,7 +37,8 @@
 // GFLOP, 51 us at the rate of a large fp32 GEMM): 94 us, against 35.5 ms on
 // the general-shape kernel. What is left is a unit's start and end (its
 // descriptor, query and slots, the masked tile, the merge: as long as eight
-// of its ~20 tiles a wave) and the last units' imbalance.
+// of its ~20 tiles a wave), the last units' imbalance, and the key loop's
+// mid-step wait for the next tile's K.
 #include "li_attention.h"
 #include "li_mfma.h"
 
@@ -99,7 +100,7 @@ __global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(
   constexpr int kStage = kH * kPlaneBytes;
   __shared__ __attribute__((aligned(1024))) union {
     char k[kF32Waves][2][kStage];
-    float acc[kF32Waves][16][D + 4];  // rows 16 bytes past a multiple of the bakF32Waves
+    float acc[kF32Waves][16][D + 4];  // rows 16 bytes past a multiple of the banks
   } lds;
   __shared__ float s_m[kF32Waves][16], s_l[kF32Waves][16];
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -299,7 +300,9 @@ __global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(
   // This wave's tiles: kb + 16 (w + 4 i). The first `clear` tiles of the
   // range are seen whole by every row; they run with slots two tiles ahead
   // of the fold and rows one. Look-ahead past the range reads the last key's
-  // slot, a real row.
+  // slot, a real row. (As compiled it reaches less far: `slot_of` narrows its
+  // load at once, and the wait for that, which the compiler places in
+  // mid-step, is also one for the next tile's K.)
   const int ntiles = ke > kb ? (ke - kb + 15) / 16 : 0;
   const int clear = max(0, min(lim_lo + 1, ke) - kb) / 16;
   auto slot_of = [&](int tile) -> int { return (int)srow[min(kb + 16 * tile + n, ke - 1)]; };
@@ -328,7 +331,7 @@ __global__ __launch_bounds__(64 * kF32Waves) __attribute__((amdgpu_waves_per_eu(
       // and one other: a step whose look-ahead nobody reads may not use this
       // count, since the compiler drops such loads.
       li_wait_vm<8 * kH + 1>();
-      // (Left to itself the scheduler sikF32Waves the loads between the MFMAs.)
+      // (Left to itself the scheduler sinks the loads between the MFMAs.)
       __builtin_amdgcn_sched_barrier(0);
       fold(std::false_type{}, kst, v, s0, kb + 16 * tile);
       // The stage's reads are done before the next step's loads fill it.

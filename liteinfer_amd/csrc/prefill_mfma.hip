@@ -1703,7 +1703,8 @@ static int launch_prefill_waves(AttnArgs a, int dtype, hipStream_t s, const Attn
   // A split pass of head_dim 64 is direct too (its pieces are at most the
   // grid's units): against the list's, 30.0 -> 26.6 us for 100 queries over
   // 4,096 keys, 47.5 -> 41.8 for 512 over 4,096, 37.3 -> 30.1 for 64 over
-  // 15,000 (bf16, 32 / 8 heads). At head_dim 128 a large one loses what a
+  // 15,000, and no large one lost (1,000 over 6,000 83.3 -> 80.0, over 32,000
+  // 289 -> 274; bf16, 32 / 8 heads). At head_dim 128 a large one loses what a
   // small one gains (64 over 1,024: 33.3 -> 31.6; 1,000 over 6,000: 128.2 ->
   // 129.2), so it keeps the list.
   const bool direct =

@@ -265,10 +265,12 @@ __global__ __launch_bounds__(64 * NW) void skinny_gemm(GemmArgs a) {
 // 16 different bank groups). Eight waves, BM / 64 of them along x's rows and
 // the rest along N, each 64 rows by BN / 16 / kWn groups of 16 outputs.
 //
-// Its bound is what a CU loads: 28672 x 4096 at 256 rows takes 71 us with the
-// loads alone (3.1 MB a CU, 44 GB/s; 66 without those of x, 63 without those of
-// W), 55 with the LDS reads and products alone, 78 whole; hence the rule in
-// cut_of.
+// Its loads set its pace: 28672 x 4096 at 256 rows takes 71 us with the loads
+// alone (3.1 MB a CU, 44 GB/s; 66 without those of x, 63 without those of W),
+// 55 with the LDS reads and products alone, 78 whole; hence the rule in
+// cut_of. That is with the wait below, which holds the 256-row kernels to 32
+// KB in flight a CU where their rings would allow 64 (48 in 64-row tiles): not
+// what a CU can load.
 template <typename T, int BM, int BN, int RX, int RW, bool kGate>
 __global__ __launch_bounds__(512) void batch_gemm(GemmArgs a) {
   using M = Mfma<T>;
@@ -366,7 +368,9 @@ __global__ __launch_bounds__(512) void batch_gemm(GemmArgs a) {
   for (int st = 0; st < ns; ++st) {
     // Loads newer than both W st and x st: in the first two stages those of W
     // st + 1 .. st + RW - 2 (x 0 and x 1 are older); later W st + RW - 3, x st
-    // + 1 and W st + RW - 2; near the end at least x st + 1.
+    // + 1 and W st + RW - 2; near the end at least x st + 1. One count serves
+    // both: with 256 rows it is the first two stages', stricter than the
+    // others need (4 against 8, in 64-row tiles 4 against 6).
     constexpr int kNewer = (RW - 2) * kWi < 2 * kWi + kXi ? (RW - 2) * kWi : 2 * kWi + kXi;
     if (st + RW - 1 < ns) li_wait_vm<kNewer>();
     else if (st >= 2 && st + 1 < ns) li_wait_vm<kXi>();
